@@ -448,9 +448,9 @@ def main() -> int:
     unit = 2.0 * hq * d * pairs          # FLOP of one GEMM over the visible pairs
     total_flops = 7.0 * unit            # fwd (2 GEMMs) + bwd (5 GEMMs)
     value = total_flops / (ms_per_step * 1e-3) / 1e12
-    # the SIMT kernels compute in fp32 on the vector ALUs, whatever the I/O dtype
+    # the general kernels are priced against fp32: the fp32 MFMA, or (bf16) bf16 MFMAs that carry fp32 P and dS
     peak = BF16_PEAK_TFLOPS if plan.path == "mfma" else FP32_PEAK_TFLOPS
-    prefix = {"32x32x16": "tpr::mfma_", "16x16x32": "tpr::m16_", None: "tpr::simt_"}[plan.mfma_shape]
+    prefix = {"32x32x16": "tpr::mfma_", "16x16x32": "tpr::m16_", None: "tpr::gen_"}[plan.mfma_shape]
     # executed MFMA work per kernel: the forward 2 GEMMs, dK/dV 4; dQ 1 from
     # the dS store, 3 when it recomputes S and dP
     kernels = {

@@ -30,13 +30,16 @@ ARCH = os.environ.get("TPR_OFFLOAD_ARCH", "gfx950")
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 HIP_UNITS = [
     ("tpr_abi.hip", "tpr_abi", []),
-    ("tpr_simt.hip", "tpr_simt", []),
     ("tpr_mfma.hip", "tpr_mfma", []),
     ("tpr_mfma16.hip", "tpr_mfma16_d64", ["-DTPR_M16_HEAD_DIM=64", "-DTPR_M16_GROUP=7", *_VGPR_FORM]),
     ("tpr_mfma16.hip", "tpr_mfma16_d256_fwd", ["-DTPR_M16_HEAD_DIM=256", "-DTPR_M16_GROUP=1", *_VGPR_FORM]),
     ("tpr_mfma16.hip", "tpr_mfma16_d256_dkdv", ["-DTPR_M16_HEAD_DIM=256", "-DTPR_M16_GROUP=2", *_VGPR_FORM]),
     ("tpr_mfma16.hip", "tpr_mfma16_d256_dq", ["-DTPR_M16_HEAD_DIM=256", "-DTPR_M16_GROUP=4"]),
 ]
+# the general family: (fp32?, padded head size)
+GEN_UNITS = [(1, 64), (1, 128), (1, 256), (0, 64), (0, 96), (0, 128), (0, 256)]
+HIP_UNITS += [("tpr_gen.hip", f"tpr_gen_{'f32' if f else 'bf16'}_{dp}",
+               [f"-DTPR_GEN_FP32={f}", f"-DTPR_GEN_DP={dp}"]) for f, dp in GEN_UNITS]
 CXX_SOURCES = ["tpr_plan.cpp"]
 
 

@@ -24,7 +24,7 @@ TPR_DTYPE_BF16 = 0
 TPR_DTYPE_FP32 = 1
 
 TPR_PLAN_RECOMPUTE_DQ = 1
-TPR_PLAN_MASKED = 2                       # plan for calls with a physical key mask (SIMT kernels)
+TPR_PLAN_MASKED = 2                       # plan for calls with a physical key mask (general kernels)
 TPR_DS_STORE_DEFAULT = -1                 # TprTreeDesc.ds_store_max_bytes: the library's default budget
 TPR_DS_STORE_DEFAULT_BYTES = 8 << 30      # ... which is 8 GiB
 

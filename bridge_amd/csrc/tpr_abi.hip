@@ -13,9 +13,38 @@
 
 namespace tpr {
 
-int launch_simt_fwd(const KernelArgs& a, bool fp32, hipStream_t s);
-int launch_delta(const KernelArgs& a, bool fp32, hipStream_t s);
-int launch_simt_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, bool fp32, hipStream_t s);
+// the general family (tpr_gen.hip), one object per type and padded head size:
+// forward or dQ over a.n_items work items, dK/dV tiles, delta
+#define TPR_GEN_UNITS(X) X(f32, 64) X(f32, 128) X(f32, 256) X(bf16, 64) X(bf16, 96) X(bf16, 128) X(bf16, 256)
+#define X(t, dp)                                                                       \
+  int launch_gen_query_##t##_##dp(const KernelArgs& a, bool dq, hipStream_t s);        \
+  int launch_gen_dkdv_##t##_##dp(const KernelArgs& a, int n_dkdv, hipStream_t s);      \
+  int launch_gen_delta_##t##_##dp(const KernelArgs& a, hipStream_t s);
+TPR_GEN_UNITS(X)
+#undef X
+struct GenUnit {
+  int (*query)(const KernelArgs&, bool, hipStream_t);
+  int (*dkdv)(const KernelArgs&, int, hipStream_t);
+  int (*delta)(const KernelArgs&, hipStream_t);
+};
+inline GenUnit gen_unit(bool fp32, int d) {
+  const int key = (fp32 ? 1000 : 0) + gen_dp(fp32, d);
+#define TPR_GEN_KEY_f32 1000
+#define TPR_GEN_KEY_bf16 0
+#define X(t, dp) \
+  if (key == TPR_GEN_KEY_##t + dp) return {launch_gen_query_##t##_##dp, launch_gen_dkdv_##t##_##dp, launch_gen_delta_##t##_##dp};
+  TPR_GEN_UNITS(X)
+#undef X
+  return {};  // not reached: gen_dp() gives the sizes listed
+}
+// dK/dV tiles, then dQ
+inline int launch_gen_bwd(KernelArgs a, int n_fwd, int n_dkdv, bool fp32, hipStream_t s) {
+  const GenUnit u = gen_unit(fp32, a.d);
+  const int rc = u.dkdv(a, n_dkdv, s);
+  if (rc != 0) return rc;
+  a.n_items = n_fwd;
+  return u.query(a, true, s);
+}
 int launch_mfma_fwd(const KernelArgs& a, hipStream_t s);
 int launch_mfma_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, int n_red, hipStream_t s);
 int launch_mfma_delta(const KernelArgs& a, hipStream_t s);
@@ -70,7 +99,8 @@ KernelArgs args_from_plan(const int32_t* ph, const int32_t* pd, float scale) {
   a.d = ph[PF_D];
   a.group = a.hq / a.hkv;
   // query heads per forward / dQ workgroup: gcd(group, waves per workgroup)
-  const int waves = ph[PF_PATH] == PATH_MFMA16 ? kM16Waves : kFwdWaves;
+  a.split = ph[PF_PATH] == PATH_GEN ? ph[PF_SPLIT] : 1;
+  const int waves = ph[PF_PATH] == PATH_MFMA16 ? kM16Waves : ph[PF_PATH] == PATH_GEN ? (a.split == 1 ? kGenWaves : 1) : kFwdWaves;
   a.hpw = 1;
   for (int g = waves; g >= 1; g--)
     if (a.group % g == 0 && waves % g == 0) { a.hpw = g; break; }
@@ -171,7 +201,7 @@ namespace {
 // floats of one stat row set of the MFMA backward ([Hq, Tq] padded to a
 // multiple of 64, so every area after it stays 256-byte aligned)
 size_t stat_row_floats(const int32_t* ph) {
-  if (ph[PF_PATH] == PATH_SIMT || ph[PF_TOTAL_Q] <= 0) return 0;
+  if (ph[PF_PATH] == PATH_GEN || ph[PF_TOTAL_Q] <= 0) return 0;
   const size_t rows = static_cast<size_t>(ph[PF_HQ]) * static_cast<size_t>(ph[PF_TOTAL_Q]);
   return (rows + 63) / 64 * 64;
 }
@@ -214,7 +244,7 @@ extern "C" int tpr_attn_fwd(const TprFwdParams* p, void* stream) {
   if (rc) return rc;
   if ((rc = check_scale(p->softmax_scale))) return rc;
   const int32_t* ph = p->plan_host;
-  const bool mfma = ph[PF_PATH] != PATH_SIMT;  // either MFMA family: 16-byte aligned rows
+  const bool mfma = ph[PF_PATH] != PATH_GEN;  // either MFMA family: 16-byte aligned rows
   const bool any_q = ph[PF_TOTAL_Q] > 0, any_p = ph[PF_TOTAL_PREFIX] > 0;
   if ((rc = check_tensor(p->q, "q", any_q, mfma)) || (rc = check_tensor(p->k, "k", any_q, mfma)) ||
       (rc = check_tensor(p->v, "v", any_q, mfma)) || (rc = check_tensor(p->out, "out", any_q, mfma)) ||
@@ -236,7 +266,7 @@ extern "C" int tpr_attn_fwd(const TprFwdParams* p, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   rc = ph[PF_PATH] == PATH_MFMA     ? launch_mfma_fwd(a, s)
        : ph[PF_PATH] == PATH_MFMA16 ? launch_m16_fwd(a, s)
-                                    : launch_simt_fwd(a, ph[PF_DTYPE] == TPR_DTYPE_FP32, s);
+                                    : gen_unit(ph[PF_DTYPE] == TPR_DTYPE_FP32, a.d).query(a, false, s);
   if (rc) return fail(TPR_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(hipGetLastError()));
   return TPR_OK;
 }
@@ -264,7 +294,7 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
     return fail(TPR_ERR_INVALID_ARGUMENT, "flags must be 0 or TPR_BWD_ACCUMULATE_PREFIX_F32, got %d", p->flags);
   const int32_t* ph = p->plan_host;
   const int path = ph[PF_PATH];
-  const bool mfma = path != PATH_SIMT;  // either MFMA family: 16-byte aligned rows
+  const bool mfma = path != PATH_GEN;  // either MFMA family: 16-byte aligned rows
   const bool any_q = ph[PF_TOTAL_Q] > 0, any_p = ph[PF_TOTAL_PREFIX] > 0;
   if ((rc = check_tensor(p->q, "q", any_q, mfma)) || (rc = check_tensor(p->k, "k", any_q, mfma)) ||
       (rc = check_tensor(p->v, "v", any_q, mfma)) || (rc = check_tensor(p->out, "out", any_q, mfma)) ||
@@ -312,16 +342,16 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
   const bool fp32 = ph[PF_DTYPE] == TPR_DTYPE_FP32;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int n_dkdv = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) ? ph[PF_N_DKDV] : 0;
-  const int n_red = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[PF_N_RED] : 0;  // 0 on the SIMT path
+  const int n_red = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[PF_N_RED] : 0;  // 0 on the general path
   // dQ work items: the forward's, or a dS-store plan's own list
   const int n_dq = (phases & TPR_BWD_DQ) ? (ph[PF_N_DQS] > 0 ? ph[PF_N_DQS] : ph[PF_N_FWD]) : 0;
   if (phases & TPR_BWD_DELTA)
     rc = path == PATH_MFMA ? launch_mfma_delta(a, s) : path == PATH_MFMA16 ? launch_m16_delta(a, s)
-                                                                          : launch_delta(a, fp32, s);
+                                                                          : gen_unit(fp32, a.d).delta(a, s);
   if (!rc && (n_dkdv || n_red || n_dq))
     rc = path == PATH_MFMA     ? launch_mfma_bwd(a, n_dq, n_dkdv, n_red, s)
          : path == PATH_MFMA16 ? launch_m16_bwd(a, n_dq, n_dkdv, n_red, s)
-                               : launch_simt_bwd(a, n_dq, n_dkdv, fp32, s);
+                               : launch_gen_bwd(a, n_dq, n_dkdv, fp32, s);
   if (rc) return fail(TPR_ERR_LAUNCH, "backward launch failed: %s", hipGetErrorString(hipGetLastError()));
   return TPR_OK;
 }

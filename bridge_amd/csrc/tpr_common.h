@@ -9,7 +9,7 @@
 namespace tpr {
 
 constexpr int32_t kPlanMagic = 0x31525054;  // "TPR1"
-constexpr int32_t kPlanVersion = 7;
+constexpr int32_t kPlanVersion = 8;
 
 // Header word indices.
 enum PlanField : int {
@@ -55,11 +55,13 @@ enum PlanField : int {
   PF_N_DQS,          // dQ work items of a dS-store plan (0: dQ takes the forward items)
   PF_OFF_DQS,        // [n][4] like the forward items: 8 waves of kDqsTokens (head_dim 128) or
                      // kM16Tokens (head_dim 256) tokens each
+  PF_SPLIT,          // general kernels: waves that share a forward / dQ row block, each taking
+                     // every PF_SPLIT-th key tile (1, or gen_split())
   PF_HEADER_WORDS = 40
 };
 
 enum KernelPath : int32_t {
-  PATH_SIMT = 0,    // fp32-accumulate SIMT kernels (fp32, or bf16 with another head_dim)
+  PATH_GEN = 0,     // general MFMA kernels (fp32; bf16 with another head_dim; key masks)
   PATH_MFMA = 1,    // bf16 MFMA kernels, head_dim 128 (32x32x16 MFMA)
   PATH_MFMA16 = 2   // bf16 MFMA kernels, head_dim 64 or 256 (16x16x32 MFMA)
 };
@@ -93,10 +95,15 @@ enum RedField : int {
 };
 
 // ---- tile shapes -----------------------------------------------------------
-// SIMT family (fp32, or bf16 with head_dim != 128; head_dim a multiple of 8, at most 256)
-constexpr int kSimtQ = 64;      // queries per forward / dQ block (one head)
-constexpr int kSimtKeys = 64;   // keys per dK/dV block
-constexpr int kSimtTile = 32;   // keys (fwd/dQ) or queries (dK/dV) staged per LDS tile
+// General family (fp32, bf16 with a head_dim the others do not cover, key
+// masks; head_dim a multiple of 8, at most 256)
+constexpr int kGenRows = 32;    // rows per tile, and rows a wave owns
+constexpr int kGenWaves = 4;    // row blocks (waves) per forward / dQ workgroup without a split
+constexpr int kGenKeys = 64;    // keys per dK/dV workgroup
+// padded head size of the kernels that serve head_dim d
+constexpr int gen_dp(bool fp32, int d) { return d <= 64 ? 64 : d <= 96 && !fp32 ? 96 : d <= 128 ? 128 : 256; }
+// the other value PF_SPLIT takes: a power of two of waves whose K/V tiles are in LDS at once
+constexpr int gen_split(bool fp32, int dp) { return (fp32 ? dp == 64 ? 8 : dp == 128 ? 4 : 2 : dp <= 128 ? 8 : 4); }
 
 // MFMA family (bf16, head_dim 128)
 constexpr int kMfmaD = 128;

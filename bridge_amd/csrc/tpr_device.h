@@ -43,7 +43,8 @@ struct KernelArgs {
   int32_t acc_prefix;  // dpk/dpv are fp32 accumulators: add the prefix gradient instead of writing it
   float scale;
   int32_t hq, hkv, d, group;
-  int32_t hpw;  // query heads per forward/dQ workgroup (MFMA path)
+  int32_t hpw;  // query heads per forward/dQ workgroup
+  int32_t split;  // general kernels: waves per forward/dQ row block
   int32_t total_q, total_prefix, max_depth;
   int32_t off_cu, off_node_off, off_anc, off_node_leaf;
   int32_t off_qblk, off_leaf_qblk, off_fwd, off_dkdv, off_red;
@@ -67,7 +68,7 @@ struct KernelArgs {
   // the head_dim-256 dQ-from-store work items (PF_OFF_DQS) and their query
   // heads per workgroup
   int32_t off_dqs, hpw_dqs;
-  // physical key mask of a masked plan (SIMT kernels): nonzero = hidden; row
+  // physical key mask of a masked plan (general kernels): nonzero = hidden; row
   // = query row of q, column = key position in the row's leaf key sequence
   // (ancestor nodes root first, then the suffix)
   const uint8_t* mask;

@@ -25,6 +25,8 @@ namespace tpr {
 namespace {
 
 constexpr int kXcds = 8;
+// general kernels: row blocks below which a block's keys are split over waves
+constexpr int kGenSplitBlocks = 4 * kPlanCus;
 
 struct Item {
   std::vector<int32_t> words;
@@ -36,7 +38,8 @@ int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // Deal items into per-XCD queues and interleave; pads with empty items
 // (first word -1) so every queue has the same length.
-std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words_per_item, int32_t* count) {
+std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words_per_item, int32_t* count,
+                                    bool two_per_cu = false) {
   std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.work > b.work; });
   std::vector<std::vector<const Item*>> queue(kXcds);
   std::vector<int64_t> load(kXcds, 0);
@@ -55,6 +58,13 @@ std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words
     queue[best].push_back(&it);
     load[best] += it.work;
   }
+  // Two workgroups run on a CU at once: when a queue is no longer than its
+  // XCD's slots, the CUs' second items run beside the first ones, so the
+  // shortest go with the longest.
+  if (two_per_cu)
+    for (auto& q : queue)
+      if (q.size() > kPlanCus / kXcds && q.size() <= 2 * kPlanCus / kXcds)
+        std::reverse(q.begin() + kPlanCus / kXcds, q.end());
   size_t depth = 0;
   for (auto& q : queue) depth = std::max(depth, q.size());
   std::vector<int32_t> out;
@@ -145,13 +155,13 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
                   "descendant leaves of node %d are not contiguous; number leaves in DFS order", n);
   }
 
-  // a masked plan runs the SIMT kernels, the ones that read a key mask
+  // a masked plan runs the general kernels, the ones that read a key mask
   const bool masked = (t->flags & TPR_PLAN_MASKED) != 0;
-  const int path = t->dtype != TPR_DTYPE_BF16 || masked ? PATH_SIMT
+  const int path = t->dtype != TPR_DTYPE_BF16 || masked ? PATH_GEN
                    : D == kMfmaD             ? PATH_MFMA
                    : (D == 64 || D == 256)   ? PATH_MFMA16
-                                             : PATH_SIMT;
-  const bool mfma_family = path != PATH_SIMT;
+                                             : PATH_GEN;
+  const bool mfma_family = path != PATH_GEN;  // the tuned bf16 families
   const int G = Hq / Hkv;
   std::vector<int64_t> prefix_len(N, 0);
   for (int s = 0; s < N; s++)
@@ -198,7 +208,7 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
     std::copy(leaf_runs[s].begin(), leaf_runs[s].end(), runs_flat.begin() + static_cast<size_t>(s) * run_words);
 
   // ---- query-block list (dK/dV granularity) --------------------------------
-  const int BQ = mfma_family ? kDkdvQ : kSimtTile;
+  const int BQ = mfma_family ? kDkdvQ : kGenRows;
   std::vector<int32_t> qblk, leaf_qblk(N + 1, 0);
   for (int s = 0; s < N; s++) {
     leaf_qblk[s] = static_cast<int32_t>(qblk.size() / 2);
@@ -211,7 +221,7 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   const int32_t n_qblk = leaf_qblk[N];
 
   // ---- forward / dQ items -----------------------------------------------------
-  int heads_per_wg, tokens_per_wg;
+  int heads_per_wg, tokens_per_wg, split = 1;
   if (path == PATH_MFMA) {
     heads_per_wg = gcd_int(G, kFwdWaves);
     tokens_per_wg = kFwdTokens * (kFwdWaves / heads_per_wg);
@@ -219,12 +229,22 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
     heads_per_wg = gcd_int(G, kM16Waves);
     tokens_per_wg = kM16Tokens * (kM16Waves / heads_per_wg);
   } else {
-    heads_per_wg = 1;
-    tokens_per_wg = kSimtQ;
+    // A 32-row block is one wave's work when the blocks alone give every SIMD
+    // a wave; with fewer, gen_split() waves share a block's keys (fp32, prefix
+    // 512 + 2 x 512, 4 heads, d64: forward 41 us with 4 waves a block, 26 with 8).
+    const bool fp32 = t->dtype == TPR_DTYPE_FP32;
+    int64_t blocks = 0;
+    for (int s = 0; s < N; s++) blocks += static_cast<int64_t>((cu[s + 1] - cu[s] + kGenRows - 1) / kGenRows) * Hq;
+    split = blocks < kGenSplitBlocks ? gen_split(fp32, gen_dp(fp32, D)) : 1;
+    heads_per_wg = split == 1 ? gcd_int(G, kGenWaves) : 1;
+    tokens_per_wg = split == 1 ? kGenRows * (kGenWaves / heads_per_wg) : kGenRows;
   }
   // Leaf-major order (longest leaf first, largest token blocks first within a
   // leaf): the workgroups that run together on an XCD then share one leaf's
-  // suffix K/V besides the prefix, which keeps both in its L2.
+  // suffix K/V besides the prefix, which keeps both in its L2. The general
+  // kernels are far from that bound and take the items by work alone (with
+  // the pairing of order_for_xcds, fp32 prefix 1024 + 2 x 1024, GQA 32/8,
+  // d128: forward 539 -> 413 us).
   std::vector<int> leaf_rank(N);
   {
     std::vector<int> by_len(N);
@@ -244,13 +264,13 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
         for (int qh = 0; qh < Hq; qh += heads) {
           Item it;
           it.words = {s, tok, qh, qh / G};
-          it.work = keys + static_cast<int64_t>(N - leaf_rank[s]) * (int64_t{1} << 40);
+          it.work = keys + (mfma_family ? static_cast<int64_t>(N - leaf_rank[s]) * (int64_t{1} << 40) : 0);
           it.kvh = qh / G;
           items.push_back(std::move(it));
         }
       }
     }
-    return order_for_xcds(items, Hkv, 4, count);
+    return order_for_xcds(items, Hkv, 4, count, path == PATH_GEN && split == 1);
   };
   int32_t n_fwd = 0;
   std::vector<int32_t> fwd_words = query_items(heads_per_wg, tokens_per_wg, &n_fwd);
@@ -264,7 +284,7 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   // chunks that each write an fp32 partial, summed afterwards in chunk (=
   // leaf) order by a reduction item. Ranges that fit stay whole: no partials
   // and no reduction.
-  const int KT = path == PATH_MFMA ? kDkdvKeys : path == PATH_MFMA16 ? m16_keys(D) : kSimtKeys;
+  const int KT = path == PATH_MFMA ? kDkdvKeys : path == PATH_MFMA16 ? m16_keys(D) : kGenKeys;
   int prefix_cap = kDkdvPrefixChunk;
   if (mfma_family) {
     int64_t total = 0;  // query blocks streamed over all (tile, KV head) items
@@ -451,6 +471,7 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   plan[PF_DS_SLOTS] = static_cast<int32_t>(ds_slots);
   plan[PF_OFF_DS] = ds_table.empty() ? 0 : append(ds_table.data(), ds_table.size());
   plan[PF_MASK_COLS] = static_cast<int32_t>(mask_cols);
+  plan[PF_SPLIT] = split;
   plan[PF_N_DQS] = n_dqs;
   plan[PF_OFF_DQS] = dqs_words.empty() ? 0 : append(dqs_words.data(), dqs_words.size());
   plan[PF_TOTAL_WORDS] = static_cast<int32_t>(plan.size());

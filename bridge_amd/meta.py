@@ -62,7 +62,8 @@ class LaunchPlan:
     @property
     def path(self) -> str:
         """Kernel path: "mfma" (bf16 matrix-core kernels: head_dim 64, 128 and
-        256) or "simt" (fp32, and bf16 with other head sizes)."""
+        256) or "simt", the general kernels (fp32, bf16 with other head sizes,
+        key masks; the name dates from their vector-ALU form)."""
         return "mfma" if int(self.host[_PF_PATH]) in (1, 2) else "simt"
 
     @property
@@ -82,7 +83,7 @@ class LaunchPlan:
     @property
     def masked(self) -> bool:
         """Whether the plan is for calls with a physical key mask (built with
-        ``masked=True``; SIMT kernels, the mask the only visibility rule)."""
+        ``masked=True``; general kernels, the mask the only visibility rule)."""
         return int(self.host[_PF_MASK_COLS]) > 0
 
     @property
@@ -240,7 +241,7 @@ class TPRPrefixMeta:
 
         ``masked=True``: the plan for calls that pass a physical key mask,
         which is then the only visibility rule (the reference's custom-mask
-        mode); it runs the SIMT kernels, for any dtype and head size, with
+        mode); it runs the general kernels, for any dtype and head size, with
         no dS store."""
         if dtype == torch.bfloat16:
             code = _lib.TPR_DTYPE_BF16

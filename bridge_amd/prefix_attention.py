@@ -24,7 +24,7 @@ rectangular_causal_attention(q, cat(prefix_k, k), cat(prefix_v, v))
 causal rule by a physical key mask, the reference's custom-mask mode
 (rectangular_attention.py:112-122): row r is query row r, column c is key c
 of that row's leaf key sequence cat(ancestor nodes root first, own suffix),
-and L is at least ``meta.max_keys()``. Masked calls run on the SIMT kernels.
+and L is at least ``meta.max_keys()``. Masked calls run on the general kernels.
 A query row that sees no key gets output 0 and zero gradients.
 """
 

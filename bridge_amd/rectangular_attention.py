@@ -16,7 +16,7 @@ reference's caller builds them (attention.py:150-158): the prefix length is
 A physical ``attention_mask`` (bool ``[Sq, Skv]``, True = excluded) is the
 sole visibility rule, as in the reference's custom-mask mode (sparse mode 0
 with the token window open, :112-122): it may hide padding rows and columns
-or show more than the causal mask. It runs on the masked (SIMT) kernels,
+or show more than the causal mask. It runs on the masked (general) kernels,
 except a mask equal to the right-down causal one, which takes the unmasked
 kernels. A query row the mask hides entirely gets output 0 and no gradient.
 """

@@ -58,8 +58,8 @@ typedef enum TprStatus {
 
 /* head_dim: a multiple of 8, at most 256. bf16 with head_dim 128 runs on the
  * 32x32x16 MFMA kernels, bf16 with head_dim 64 or 256 on the 16x16x32 MFMA
- * kernels (any tree depth); fp32 and the other head sizes on the SIMT
- * kernels. All accumulate in fp32. */
+ * kernels (any tree depth); fp32 and the other head sizes on the
+ * general MFMA kernels. All accumulate in fp32. */
 typedef enum TprDtype {
   TPR_DTYPE_BF16 = 0, /* bf16 in/out, fp32 accumulation */
   TPR_DTYPE_FP32 = 1  /* fp32 in/out, fp32 accumulation */
@@ -98,7 +98,7 @@ typedef enum TprDtype {
  * mask (TprFwdParams.mask): the mask is then the only visibility rule, as in
  * the reference's custom-mask mode (sparse mode 0, rectangular_attention.py:
  * 112-122) -- the causal rule is not applied on top of it, so a mask may also
- * show a leaf's later suffix keys. Such a plan always runs the SIMT kernels
+ * show a leaf's later suffix keys. Such a plan always runs the general kernels
  * (any dtype and head size), with no dS store; every call with it must pass a
  * mask, and a call with a mask must use such a plan.
  * flags: 0 or an OR of TPR_PLAN_RECOMPUTE_DQ and TPR_PLAN_MASKED. */
