@@ -30,7 +30,9 @@ ARCH = os.environ.get("TPR_OFFLOAD_ARCH", "gfx950")
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 HIP_UNITS = [
     ("tpr_abi.hip", "tpr_abi", []),
-    ("tpr_mfma.hip", "tpr_mfma", []),
+    ("tpr_mfma.hip", "tpr_mfma_fwd", ["-DTPR_MFMA_GROUP=1"]),
+    ("tpr_mfma.hip", "tpr_mfma_dkdv", ["-DTPR_MFMA_GROUP=2"]),
+    ("tpr_mfma.hip", "tpr_mfma_dq", ["-DTPR_MFMA_GROUP=4"]),
     ("tpr_mfma16.hip", "tpr_mfma16_d64", ["-DTPR_M16_HEAD_DIM=64", "-DTPR_M16_GROUP=7", *_VGPR_FORM]),
     ("tpr_mfma16.hip", "tpr_mfma16_d256_fwd", ["-DTPR_M16_HEAD_DIM=256", "-DTPR_M16_GROUP=1", *_VGPR_FORM]),
     ("tpr_mfma16.hip", "tpr_mfma16_d256_dkdv", ["-DTPR_M16_HEAD_DIM=256", "-DTPR_M16_GROUP=2", *_VGPR_FORM]),

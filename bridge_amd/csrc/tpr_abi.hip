@@ -46,8 +46,13 @@ inline int launch_gen_bwd(KernelArgs a, int n_fwd, int n_dkdv, bool fp32, hipStr
   return u.query(a, true, s);
 }
 int launch_mfma_fwd(const KernelArgs& a, hipStream_t s);
-int launch_mfma_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, int n_red, hipStream_t s);
+int launch_mfma_dkdv(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s);
+int launch_mfma_dq(const KernelArgs& a, int n_fwd, hipStream_t s);
 int launch_mfma_delta(const KernelArgs& a, hipStream_t s);
+inline int launch_mfma_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, int n_red, hipStream_t s) {
+  const int rc = launch_mfma_dkdv(a, n_dkdv, n_red, s);
+  return rc != 0 ? rc : launch_mfma_dq(a, n_fwd, s);
+}
 // the 16x16x32 family (tpr_mfma16.hip), one object per head size and kernel group
 int launch_m16_fwd_d64(const KernelArgs& a, hipStream_t s);
 int launch_m16_fwd_d256(const KernelArgs& a, hipStream_t s);

@@ -25,9 +25,16 @@
 // operand straight from registers, and V is read column-wise from its
 // row-major LDS tile with ds_read_tr16_b64.
 
+// The file is compiled once per kernel group (TPR_MFMA_GROUP bits: 1 = forward
+// and delta, 2 = dK/dV and its reduction, 4 = dQ).
+
 #include <type_traits>
 
 #include "tpr_kernel_util.h"
+
+#ifndef TPR_MFMA_GROUP
+#define TPR_MFMA_GROUP 7
+#endif
 
 namespace tpr {
 namespace {
@@ -225,6 +232,7 @@ __device__ __forceinline__ void store_tile_rows(char* stage, const f32x16 (&acc)
   }
 }
 
+#if TPR_MFMA_GROUP & 1
 // ---------------------------------------------------------------------------
 // Forward
 //
@@ -255,10 +263,6 @@ __device__ __forceinline__ void qk_tile(const char* kt, const bf16x8 (&qv)[8], c
 // so unscaled probabilities stay <= 2^8 (exact arithmetic, fp32/bf16 safe).
 constexpr float kRescaleSlack = 8.f;
 
-// dK/dV: S and dP MFMAs written as asm with their accumulators in VGPRs
-#ifndef TPR_DKDV_VGPR_SP
-#define TPR_DKDV_VGPR_SP 1
-#endif
 #ifndef TPR_MPHASE_AHEAD
 #define TPR_MPHASE_AHEAD 4
 #endif
@@ -589,6 +593,9 @@ __global__ __launch_bounds__(256) void mfma_delta(KernelArgs a) {
   }
 }
 
+#endif  // forward, delta
+
+#if TPR_MFMA_GROUP & 4
 // ---------------------------------------------------------------------------
 // dQ: same workgroup shape, key stream and two-group ping-pong as the forward.
 //   M(j): dQ^T += K[j]^T dS^T[j], S^T[j+1] = K[j+1] Q^T, dP^T[j+1] = V[j+1] dO^T
@@ -1172,6 +1179,9 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
                       qstride, len - tw0 - 32 * j, lane);
 }
 
+#endif  // dQ
+
+#if TPR_MFMA_GROUP & 2
 // ---------------------------------------------------------------------------
 // dK/dV
 //   S = Q K^T (query rows permuted by sigma32), P = exp(scale S - lse),
@@ -1190,6 +1200,10 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
 #endif
 #ifndef TPR_DS_STORE_K2
 #define TPR_DS_STORE_K2 28
+#endif
+// dK/dV: S and dP MFMAs written as asm with their accumulators in VGPRs
+#ifndef TPR_DKDV_VGPR_SP
+#define TPR_DKDV_VGPR_SP 1
 #endif
 #ifndef TPR_DKDV_INTERLEAVE
 #define TPR_DKDV_INTERLEAVE 1
@@ -1641,21 +1655,31 @@ __global__ __launch_bounds__(256) void mfma_dkdv(KernelArgs a) {
         }
       } else if (prefix && a.acc_prefix) {
         // fp32 relay accumulators: add this (unsplit) tile's gradient, the scaled
-        // product rounded as the ordinary path rounds it, then one add (no fma)
+        // product rounded as the ordinary path rounds it, then one add (no fma).
+        // Every old value of a tensor is read before the first is written: reads
+        // behind writes that may alias them waited row by row (35 -> 24 us at
+        // prefix 1500 + 100, 600 -> 582 us at 4096 + 3590, GQA 32/8).
+        auto add_rows = [&](float* base, const f32x16 (&acc)[4], float mul) __attribute__((always_inline)) {
 #pragma clang fp contract(off)
-        float* dkf = static_cast<float*>(a.dpk);
-        float* dvf = static_cast<float*>(a.dpv);
+          float old[16][4];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int key = kw0 + 8 * (r >> 2) + 4 * h + (r & 3);
-          if (key >= seg_len) continue;
-          const int64_t off = static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kMfmaD + n;
+          for (int r = 0; r < 16; r++) {
+            const int key = min(kw0 + 8 * (r >> 2) + 4 * h + (r & 3), seg_len - 1);
+            const float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kMfmaD + n;
 #pragma unroll
-          for (int db = 0; db < 4; db++) {
-            dkf[off + 32 * db] += dk[db][r] * a.scale;
-            dvf[off + 32 * db] += dv[db][r];
+            for (int db = 0; db < 4; db++) old[r][db] = row[32 * db];
           }
-        }
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int key = kw0 + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (key >= seg_len) continue;
+            float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kMfmaD + n;
+#pragma unroll
+            for (int db = 0; db < 4; db++) row[32 * db] = old[r][db] + acc[db][r] * mul;
+          }
+        };
+        add_rows(static_cast<float*>(a.dpk), dk, a.scale);
+        add_rows(static_cast<float*>(a.dpv), dv, 1.f);
       } else {
         bf16* dkd = static_cast<bf16*>(prefix ? a.dpk : a.dk);
         bf16* dvd = static_cast<bf16*>(prefix ? a.dpv : a.dv);
@@ -1716,12 +1740,15 @@ __global__ __launch_bounds__(256) void mfma_reduce(KernelArgs a) {
   }
 }
 
+#endif  // dK/dV
+
 // Whether any of q, k, v has rows wider than packed.
 bool strided_rows(const KernelArgs& a) {
   return a.q_rs != static_cast<int64_t>(a.hq) * kMfmaD || a.k_rs != static_cast<int64_t>(a.hkv) * kMfmaD ||
          a.v_rs != static_cast<int64_t>(a.hkv) * kMfmaD;
 }
 
+#if TPR_MFMA_GROUP & 1
 template <bool kRunList>
 void launch_fwd_tile(const KernelArgs& a, hipStream_t s) {
   if (strided_rows(a))
@@ -1729,7 +1756,9 @@ void launch_fwd_tile(const KernelArgs& a, hipStream_t s) {
   else
     hipLaunchKernelGGL((mfma_fwd<kRunList, false>), dim3(a.n_items), dim3(64 * kFwdWaves), 0, s, a);
 }
+#endif
 
+#if TPR_MFMA_GROUP & 2
 template <int kHeads>
 void launch_dkdv_heads(const KernelArgs& a, int n_dkdv, hipStream_t s) {
   const bool st = strided_rows(a), ds = a.ds != nullptr;
@@ -1742,7 +1771,9 @@ void launch_dkdv_heads(const KernelArgs& a, int n_dkdv, hipStream_t s) {
   else
     hipLaunchKernelGGL((mfma_dkdv<kHeads, false, false>), dim3(n_dkdv), dim3(256), 0, s, a);
 }
+#endif
 
+#if TPR_MFMA_GROUP & 4
 template <bool kRunList>
 void launch_dq_tile(const KernelArgs& a, int n_fwd, hipStream_t s) {
   if (strided_rows(a))
@@ -1750,9 +1781,11 @@ void launch_dq_tile(const KernelArgs& a, int n_fwd, hipStream_t s) {
   else
     hipLaunchKernelGGL((mfma_dq<kRunList, false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
 }
+#endif
 
 }  // namespace
 
+#if TPR_MFMA_GROUP & 1
 int launch_mfma_fwd(const KernelArgs& a, hipStream_t s) {
   if (a.n_items > 0) {
     if (a.max_runs > kMfmaRegRuns)
@@ -1768,8 +1801,11 @@ int launch_mfma_delta(const KernelArgs& a, hipStream_t s) {
   if (blocks > 0 && a.hq > 0) hipLaunchKernelGGL(mfma_delta, dim3(blocks, a.hq), dim3(256), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
+#endif
 
-int launch_mfma_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, int n_red, hipStream_t s) {
+#if TPR_MFMA_GROUP & 2
+// dK/dV tiles, then their reduction
+int launch_mfma_dkdv(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s) {
   if (n_dkdv > 0) {
     if (a.group % 2 == 0)
       launch_dkdv_heads<2>(a, n_dkdv, s);
@@ -1781,18 +1817,23 @@ int launch_mfma_bwd(const KernelArgs& a, int n_fwd, int n_dkdv, int n_red, hipSt
     hipLaunchKernelGGL(mfma_reduce, dim3(n_red), dim3(256), 0, s, a);
     if (hipGetLastError() != hipSuccess) return 4;
   }
-  if (n_fwd > 0) {
-    if (a.ds && strided_rows(a))
-      hipLaunchKernelGGL((mfma_dqs<true>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
-    else if (a.ds)
-      hipLaunchKernelGGL((mfma_dqs<false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
-    else if (a.max_runs > kMfmaRegRuns)
-      launch_dq_tile<true>(a, n_fwd, s);
-    else
-      launch_dq_tile<false>(a, n_fwd, s);
-    if (hipGetLastError() != hipSuccess) return 4;
-  }
   return 0;
 }
+#endif
+
+#if TPR_MFMA_GROUP & 4
+int launch_mfma_dq(const KernelArgs& a, int n_fwd, hipStream_t s) {
+  if (n_fwd <= 0) return 0;
+  if (a.ds && strided_rows(a))
+    hipLaunchKernelGGL((mfma_dqs<true>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
+  else if (a.ds)
+    hipLaunchKernelGGL((mfma_dqs<false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
+  else if (a.max_runs > kMfmaRegRuns)
+    launch_dq_tile<true>(a, n_fwd, s);
+  else
+    launch_dq_tile<false>(a, n_fwd, s);
+  return hipGetLastError() == hipSuccess ? 0 : 4;
+}
+#endif
 
 }  // namespace tpr

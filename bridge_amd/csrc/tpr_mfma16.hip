@@ -1138,22 +1138,33 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
             }
           }
       } else if (prefix && a.acc_prefix) {
+        // a tensor's old values are all read before the first is written (reads
+        // behind writes that may alias them would wait row by row)
+        auto add_rows = [&](float* base, const f32x4 (&acc)[KB][T::ND], float mul) __attribute__((always_inline)) {
 #pragma clang fp contract(off)
-        float* dkf = static_cast<float*>(a.dpk);
-        float* dvf = static_cast<float*>(a.dpv);
+          float old[KB][4][T::ND];
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++)
+          for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int key = kw0 + 16 * kb + 4 * g + r;
-            if (key >= seg_len) continue;
-            const int64_t off = static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
+            for (int r = 0; r < 4; r++) {
+              const int key = min(kw0 + 16 * kb + 4 * g + r, seg_len - 1);
+              const float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
 #pragma unroll
-            for (int db = 0; db < T::ND; db++) {
-              dkf[off + 16 * db] += dk[kb][db][r] * a.scale;
-              dvf[off + 16 * db] += dv[kb][db][r];
+              for (int db = 0; db < T::ND; db++) old[kb][r][db] = row[16 * db];
             }
-          }
+#pragma unroll
+          for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const int key = kw0 + 16 * kb + 4 * g + r;
+              if (key >= seg_len) continue;
+              float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
+#pragma unroll
+              for (int db = 0; db < T::ND; db++) row[16 * db] = old[kb][r][db] + acc[kb][db][r] * mul;
+            }
+        };
+        add_rows(static_cast<float*>(a.dpk), dk, a.scale);
+        add_rows(static_cast<float*>(a.dpv), dv, 1.f);
       } else {
         bf16* dkd = static_cast<bf16*>(prefix ? a.dpk : a.dk);
         bf16* dvd = static_cast<bf16*>(prefix ? a.dpv : a.dv);
