@@ -34,6 +34,8 @@ EXPORTED_SYMBOLS = (
     "tpr_attn_plan",
     "tpr_attn_bwd_workspace_bytes",
     "tpr_attn_fwd",
+    "tpr_attn_fwd_ws",
+    "tpr_attn_fwd_workspace_bytes",
     "tpr_attn_bwd",
     "tpr_attn_bwd_phases",
     "tpr_attn_bwd_noalloc",
@@ -154,6 +156,10 @@ def load():
         lib.tpr_attn_bwd_workspace_bytes.argtypes = [_p]
         lib.tpr_attn_fwd.restype = ctypes.c_int
         lib.tpr_attn_fwd.argtypes = [ctypes.POINTER(TprFwdParams), _p]
+        lib.tpr_attn_fwd_ws.restype = ctypes.c_int
+        lib.tpr_attn_fwd_ws.argtypes = [ctypes.POINTER(TprFwdParams), _p, ctypes.c_size_t, _p]
+        lib.tpr_attn_fwd_workspace_bytes.restype = ctypes.c_size_t
+        lib.tpr_attn_fwd_workspace_bytes.argtypes = [_p]
         lib.tpr_attn_bwd.restype = ctypes.c_int
         lib.tpr_attn_bwd.argtypes = [ctypes.POINTER(TprBwdParams), _p]
         lib.tpr_attn_bwd_phases.restype = ctypes.c_int

@@ -234,12 +234,32 @@ size_t ds_bytes(const int32_t* ph) {
 }  // namespace
 }  // namespace tpr
 
+namespace tpr {
+namespace {
+// the workspace the backward cannot run without; dQ's key parts follow it
+size_t bwd_base_bytes(const int32_t* ph) { return ws_fp32_bytes(ph) + ds_bytes(ph); }
+size_t qpart_bytes(const int32_t* ph) {
+  return static_cast<size_t>(ph[PF_QSLOTS]) * qpart_slot_floats(ph[PF_PATH], ph[PF_D], ph[PF_DS_SLOTS] > 0) * sizeof(float);
+}
+size_t fpart_bytes(const int32_t* ph) {
+  return static_cast<size_t>(ph[PF_FSLOTS]) * fpart_slot_floats(ph[PF_PATH], ph[PF_D]) * sizeof(float);
+}
+}  // namespace
+}  // namespace tpr
+
 extern "C" size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host) {
   if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
-  return ws_fp32_bytes(plan_host) + ds_bytes(plan_host);
+  return bwd_base_bytes(plan_host) + qpart_bytes(plan_host);
 }
 
-extern "C" int tpr_attn_fwd(const TprFwdParams* p, void* stream) {
+extern "C" size_t tpr_attn_fwd_workspace_bytes(const int32_t* plan_host) {
+  if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
+  return fpart_bytes(plan_host);
+}
+
+extern "C" int tpr_attn_fwd(const TprFwdParams* p, void* stream) { return tpr_attn_fwd_ws(p, nullptr, 0, stream); }
+
+extern "C" int tpr_attn_fwd_ws(const TprFwdParams* p, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   if (!p) return fail(TPR_ERR_INVALID_ARGUMENT, "params must not be NULL");
   if (p->abi_version != TPR_ATTN_ABI_VERSION)
@@ -268,6 +288,17 @@ extern "C" int tpr_attn_fwd(const TprFwdParams* p, void* stream) {
   a.out = p->out;
   a.lse = p->lse;
   a.n_items = ph[PF_N_FWD];
+  if (workspace && ph[PF_N_FPART] > 0) {
+    if (workspace_bytes < fpart_bytes(ph))
+      return fail(TPR_ERR_BUFFER_TOO_SMALL, "forward workspace needs %zu bytes, got %zu", fpart_bytes(ph), workspace_bytes);
+    if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
+      return fail(TPR_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
+    a.part_ws = static_cast<float*>(workspace);
+    a.off_part = ph[PF_OFF_FPART];
+    a.n_part = ph[PF_N_FPART];
+    a.off_merge = ph[PF_OFF_FMERGE];
+    a.n_merge = ph[PF_N_FMERGE];
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   rc = ph[PF_PATH] == PATH_MFMA     ? launch_mfma_fwd(a, s)
        : ph[PF_PATH] == PATH_MFMA16 ? launch_m16_fwd(a, s)
@@ -311,7 +342,9 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
       (rc = check_tensor(p->dprefix_k, "dprefix_k", any_p, mfma)) ||
       (rc = check_tensor(p->dprefix_v, "dprefix_v", any_p, mfma)))
     return rc;
-  const size_t need = tpr_attn_bwd_workspace_bytes(ph);
+  // dQ runs in key parts where the workspace holds them too (the
+  // allocation-free backward's scratch may not)
+  const size_t need = bwd_base_bytes(ph);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return fail(TPR_ERR_BUFFER_TOO_SMALL, "backward workspace needs %zu bytes, got %zu", need, workspace_bytes);
   // the MFMA backward reads the partial slots as 16-byte vectors and DMA-copies
@@ -344,6 +377,13 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
   a.off_ds_first = ph[PF_OFF_DS] + ph[PF_NUM_NODES] + ph[PF_NUM_LEAVES];
   a.ds_slots = ph[PF_DS_SLOTS];
   a.num_nodes = ph[PF_NUM_NODES];
+  if (ph[PF_N_QPART] > 0 && workspace_bytes >= need + qpart_bytes(ph)) {
+    a.part_ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + need);
+    a.off_part = ph[PF_OFF_QPART];
+    a.n_part = ph[PF_N_QPART];
+    a.off_merge = ph[PF_OFF_QMERGE];
+    a.n_merge = ph[PF_N_QMERGE];
+  }
   const bool fp32 = ph[PF_DTYPE] == TPR_DTYPE_FP32;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int n_dkdv = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) ? ph[PF_N_DKDV] : 0;
@@ -422,7 +462,7 @@ extern "C" int tpr_attn_bwd_noalloc(const TprBwdParams* p, void* stream) {
   clear_error();
   if (!p) return fail(TPR_ERR_INVALID_ARGUMENT, "params must not be NULL");
   if (p->abi_version == TPR_ATTN_ABI_VERSION && p->plan_host && p->plan_host[PF_MAGIC] == kPlanMagic) {
-    const size_t need = tpr_attn_bwd_workspace_bytes(p->plan_host);
+    const size_t need = bwd_base_bytes(p->plan_host);
     if (need > kScratchBytes)
       return fail(TPR_ERR_UNSUPPORTED,
                   "backward workspace needs %zu bytes, more than the %zu bytes of the library's static scratch; "

@@ -57,7 +57,20 @@ enum PlanField : int {
                      // kM16Tokens (head_dim 256) tokens each
   PF_SPLIT,          // general kernels: waves that share a forward / dQ row block, each taking
                      // every PF_SPLIT-th key tile (1, or gen_split())
-  PF_HEADER_WORDS = 40
+  // Key parts: forward and dQ items whose keys are split over several
+  // workgroups, each leaving fp32 partial rows in a slot of the caller's
+  // workspace, summed afterwards in part order (0 items: no split)
+  PF_N_FPART,        // forward items [n][PT_WORDS] = PartItem
+  PF_OFF_FPART,
+  PF_N_FMERGE,       // forward items to sum [n][PT_WORDS] = PartItem (PT_SLOT first slot, PT_TILES parts)
+  PF_OFF_FMERGE,
+  PF_FSLOTS,         // forward partial slots
+  PF_N_QPART,        // the same for dQ
+  PF_OFF_QPART,
+  PF_N_QMERGE,
+  PF_OFF_QMERGE,
+  PF_QSLOTS,
+  PF_HEADER_WORDS = 48
 };
 
 enum KernelPath : int32_t {
@@ -92,6 +105,20 @@ enum RedField : int {
   RD_PAD0,
   RD_PAD1,
   RD_WORDS = 8
+};
+
+// Part item: a forward / dQ work item over tiles [PT_TILE0, + PT_TILES) of its
+// key stream.
+enum PartField : int {
+  PT_LEAF = 0,  // < 0 = empty
+  PT_TOK,
+  PT_QH,        // first query head
+  PT_KVH,
+  PT_TILE0,
+  PT_TILES,
+  PT_SLOT,      // -1: the whole stream, written directly; else partial slot
+  PT_PAD,
+  PT_WORDS = 8
 };
 
 // ---- tile shapes -----------------------------------------------------------
@@ -146,5 +173,14 @@ constexpr int ds_head_bytes(int path, int d) {
 }
 constexpr int kMfmaRegRuns = 8;       // key runs a forward / dQ workgroup holds in registers; a
                                       // launch with longer run lists reads them from the plan
+
+// fp32 partial slots of the key parts, in register order: the forward's output
+// rows then (max, sum) per row; dQ's rows
+constexpr int fpart_slot_floats(int path, int d) {
+  return (path == PATH_MFMA ? kFwdWaves * kFwdTokens : kM16Waves * kM16Tokens) * (d + 2);
+}
+constexpr int qpart_slot_floats(int path, int d, bool store) {
+  return (path == PATH_MFMA ? kFwdWaves * kDqsTokens : (store ? kM16DqsWaves : kM16Waves) * kM16Tokens) * d;
+}
 
 }  // namespace tpr

@@ -68,6 +68,10 @@ struct KernelArgs {
   // the head_dim-256 dQ-from-store work items (PF_OFF_DQS) and their query
   // heads per workgroup
   int32_t off_dqs, hpw_dqs;
+  // key parts of the forward / dQ (PF_N_FPART, PF_N_QPART): their items, the
+  // items to sum, and the partial slots (null: the unsplit items run)
+  int32_t off_part, n_part, off_merge, n_merge;
+  float* part_ws;
   // physical key mask of a masked plan (general kernels): nonzero = hidden; row
   // = query row of q, column = key position in the row's leaf key sequence
   // (ancestor nodes root first, then the suffix)

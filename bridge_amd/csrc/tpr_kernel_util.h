@@ -282,6 +282,24 @@ __device__ __forceinline__ void cursor_next(const Keys& t, Cursor& c) {
   }
 }
 
+// Steps over n tiles of the stream.
+template <typename Keys>
+__device__ __forceinline__ void cursor_skip(const Keys& t, Cursor& c, int n) {
+  while (n > 0 && c.len > 0) {
+    const int left = (c.len + kTileRows - 1) / kTileRows - c.lt;
+    if (n < left) {
+      c.lt += n;
+      return;
+    }
+    n -= left;
+    c.lt = 0;
+    do {
+      c.d++;
+      cursor_load(t, c);
+    } while (c.len == 0 && c.d < kMfmaRegRuns);
+  }
+}
+
 __device__ __forceinline__ TileLoc cursor_tile(const Cursor& c) {
   return TileLoc{static_cast<int64_t>(c.row) + c.lt * kTileRows, min(kTileRows, c.len - c.lt * kTileRows),
                  c.lt * kTileRows, c.d == 0};
@@ -341,6 +359,26 @@ __device__ __forceinline__ void kv_next(const Keys& t, const KvSources& s, KvCur
   c.k += c.kstep;
   c.v += c.vstep;
   if (c.rem <= 0) {
+    do {
+      c.d++;
+      kv_enter(t, s, c);
+    } while (c.rem == 0 && c.d < kMfmaRegRuns);
+  }
+}
+
+// Steps over n tiles of the stream.
+template <typename Keys>
+__device__ __forceinline__ void kv_skip(const Keys& t, const KvSources& s, KvCursor& c, int n) {
+  while (n > 0 && c.rem > 0) {
+    const int left = (c.rem + kTileRows - 1) / kTileRows;
+    if (n < left) {
+      c.rem -= n * kTileRows;
+      c.pos0 += n * kTileRows;
+      c.k += n * c.kstep;
+      c.v += n * c.vstep;
+      return;
+    }
+    n -= left;
     do {
       c.d++;
       kv_enter(t, s, c);

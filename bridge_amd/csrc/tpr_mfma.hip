@@ -40,6 +40,7 @@ namespace tpr {
 namespace {
 
 constexpr int kTileBytes = kTileRows * 256;   // 64 rows x 128 bf16
+constexpr int kFSlot = fpart_slot_floats(PATH_MFMA, kMfmaD), kQSlot = qpart_slot_floats(PATH_MFMA, kMfmaD, true);
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 constexpr int kBufferRsrcWord3 = 0x00020000;  // raw (untyped) buffer resource, gfx9 data format field
 constexpr int kCachePolicyNt = 2;             // buffer access cache policy: non-temporal (streaming)
@@ -271,9 +272,11 @@ constexpr int kMphaseAhead = TPR_MPHASE_AHEAD;  // LDS reads issued ahead in a f
 // kRunList: key runs read from the plan (more than kMfmaRegRuns); kStrided:
 // q, k or v rows wider than packed (the packed instance folds every row
 // stride to a constant)
-template <bool kRunList, bool kStrided>
+// kPart: items over part of their key stream (PF_OFF_FPART), for calls whose
+// query rows alone leave compute units idle
+template <bool kRunList, bool kStrided, bool kPart>
 __global__ __launch_bounds__(512) void mfma_fwd(KernelArgs a) {
-  const int32_t* item = a.plan + a.off_fwd + 4 * blockIdx.x;
+  const int32_t* item = kPart ? a.plan + a.off_part + PT_WORDS * blockIdx.x : a.plan + a.off_fwd + 4 * blockIdx.x;
   const int leaf = item[0];
   if (leaf < 0) return;
   const int tok0 = item[1], qh0 = item[2], kvh = item[3];
@@ -321,7 +324,7 @@ __global__ __launch_bounds__(512) void mfma_fwd(KernelArgs a) {
   const FwdLdsOffsets lo = make_fwd_lds_offsets(lane);
 
   const auto seg = load_keys<kRunList>(a, leaf, suffix_keys);
-  const int ntiles = seg.ntiles;
+  const int ntiles = kPart ? item[PT_TILES] : seg.ntiles;
   const KvSources src{kbase, vbase, pkbase, pvbase, k_rb, v_rb, p_rb};
   // Copy cursors. Group B copies K[0], K[1] and V[0] before the tile loop,
   // then V[j+1] at the start of its softmax phase V(j-1); group A copies
@@ -329,11 +332,12 @@ __global__ __launch_bounds__(512) void mfma_fwd(KernelArgs a) {
   // softmax phase outlasts. Both wait for their copies one phase later,
   // before the barrier ahead of the first M phase that reads them.
   KvCursor dv = kv_begin(seg, src);  // B: the next V tile
+  if constexpr (kPart) kv_skip(seg, src, dv, item[PT_TILE0]);
   if (grp) dma_tile4_fwd(dv.k, dv.krb, kv_len(dv), lds0, dl, wave & 3);  // K[0]
   KvCursor ka = dv;                  // A: the next K tile (tile 2 when the loop starts); B: tile 1 first
   if (ntiles > 1) kv_next(seg, src, ka);
   // every wave's mask cursor: the tile whose scores the next V phase masks
-  KvCursor mc = kv_begin(seg, src);
+  KvCursor mc = kPart ? dv : kv_begin(seg, src);
 
 
   f32x16 o[4];
@@ -527,6 +531,25 @@ __global__ __launch_bounds__(512) void mfma_fwd(KernelArgs a) {
 
   const float lt = wave_sum32(l);  // all 64 lanes take part in the exchange
   if (tw0 >= len) return;
+  if constexpr (kPart) {
+    const int slot = item[PT_SLOT];
+    if (slot >= 0) {
+      // partial rows, in register order (whole 1 KiB lines per store), then (m, l)
+      float* ws = a.part_ws + static_cast<int64_t>(slot) * kFSlot;
+      f32x4* po = reinterpret_cast<f32x4*>(ws) + wave * 1024 + lane;
+#pragma unroll
+      for (int db = 0; db < 4; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          po[(4 * db + g) * 64] = f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+      float* st = ws + kFwdWaves * kFwdTokens * kMfmaD + 2 * (32 * wave + n);
+      if (h == 0) {
+        st[0] = m;
+        st[1] = lt;
+      }
+      return;
+    }
+  }
   const float inv = 1.f / lt;
   if (h == 0 && t < len) a.lse[static_cast<int64_t>(head) * a.total_q + row0 + t] = m * a.scale + logf(lt);
   // O as whole non-temporal rows: cacheable stores would park the output in
@@ -536,6 +559,51 @@ __global__ __launch_bounds__(512) void mfma_fwd(KernelArgs a) {
   store_tile_rows(smem + wave * 8192, o, inv,
                   static_cast<bf16*>(a.out) + static_cast<int64_t>(row0 + tw0) * qstride + head * kMfmaD, qstride,
                   len - tw0, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Sum of the forward's key parts, part 0 first: O = sum w_p O_p / sum w_p l_p
+// with w_p = exp(m_p - max m). One wave's rows per workgroup row (blockIdx.y),
+// 32 columns per wave, four parts' loads in flight. Memory-bound: it reads the
+// partials once (34 MB in 8.7 us at prefix 8192 + 512, GQA 32/8, where the
+// parts themselves take 72 us instead of the whole items' 163).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void mfma_fwd_merge(KernelArgs a) {
+  const int32_t* item = a.plan + a.off_merge + PT_WORDS * blockIdx.x;
+  const int leaf = item[PT_LEAF];
+  const int32_t* cu = a.plan + a.off_cu;
+  const int row0 = cu[leaf], len = cu[leaf + 1] - cu[leaf];
+  const int wave = blockIdx.y, db = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
+  const int head = item[PT_QH] + wave % a.hpw, t = item[PT_TOK] + kFwdTokens * (wave / a.hpw) + n;
+  if (t >= len) return;
+  const int parts = item[PT_TILES];
+  const float* ws = a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * kFSlot;
+  const float* st = ws + kFwdWaves * kFwdTokens * kMfmaD + 2 * (32 * wave + n);
+  float m = -INFINITY;
+#pragma unroll 4
+  for (int p = 0; p < parts; p++) m = fmaxf(m, st[p * kFSlot]);
+  const float c2 = a.scale * kLog2e;
+  float l = 0.f;
+  f32x4 o[4] = {};
+#pragma unroll 4
+  for (int p = 0; p < parts; p++) {
+    const int64_t at = static_cast<int64_t>(p) * kFSlot;
+    const float w = fast_exp2((st[at] - m) * c2);
+    l += w * st[at + 1];
+    const f32x4* po = reinterpret_cast<const f32x4*>(ws + at) + wave * 1024 + 256 * db + lane;
+#pragma unroll
+    for (int g = 0; g < 4; g++) o[g] += w * po[64 * g];
+  }
+  const float inv = 1.f / l;
+  bf16* out = static_cast<bf16*>(a.out) + (static_cast<int64_t>(row0 + t) * a.hq + head) * kMfmaD + 32 * db + 4 * h;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    bf16x4 v;
+#pragma unroll
+    for (int b = 0; b < 4; b++) v[b] = static_cast<bf16>(o[g][b] * inv);
+    *reinterpret_cast<bf16x4*>(out + 8 * g) = v;
+  }
+  if (db == 0 && h == 0) a.lse[static_cast<int64_t>(head) * a.total_q + row0 + t] = m * a.scale + logf(l);
 }
 
 // ---------------------------------------------------------------------------
@@ -927,9 +995,9 @@ __global__ __launch_bounds__(512) void mfma_dq(KernelArgs a) {
 // wave's dS buffer is its own, so the dS two halves ahead is copied into it
 // as soon as the wave's reads of the current half's dS have returned.
 // ---------------------------------------------------------------------------
-template <bool kStrided>
+template <bool kStrided, bool kPart>  // as mfma_fwd; parts in 128-key tiles
 __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
-  const int32_t* item = a.plan + a.off_dqs + 4 * blockIdx.x;
+  const int32_t* item = kPart ? a.plan + a.off_part + PT_WORDS * blockIdx.x : a.plan + a.off_dqs + 4 * blockIdx.x;
   const int leaf = item[0];
   if (leaf < 0) return;
   const int tok0 = item[1], qh0 = item[2], kvh = item[3];
@@ -1028,6 +1096,7 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
       if (ckey >= clim) next_segment();
     }
   };
+  const int cend = kPart ? item[PT_TILE0] + item[PT_TILES] : 0;  // past the part's last tile
   // this wave's dS blocks: its query block's first slot, its head
   const char* ds_wave = nullptr;
   if (wave_ok) {
@@ -1052,7 +1121,7 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
     const int k0 = ckey + kTileRows * chalf;
     const bool suffix = cd == depth;
     Half t;
-    t.more = clim > 0;
+    t.more = clim > 0 && (!kPart || cpos < cend);
     t.rb = suffix ? k_rb : p_rb;
     t.k = (suffix ? kbase : pkbase) + static_cast<int64_t>(crow + k0) * t.rb;
     t.ds = ds_wave + cpos * ds_tile_bytes + 2 * chalf * 4096;
@@ -1145,6 +1214,19 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
   // ones issued are half i + 1's dS (8 blocks), and waiting until at most
   // those are outstanding means half i's K rows and dS have landed.
   next_segment();
+  if constexpr (kPart) {
+    const int tile0 = item[PT_TILE0];
+    while (cpos < tile0 && clim > 0) {
+      const int tiles = (clim + kDkdvKeys - 1) / kDkdvKeys;
+      if (tile0 - cpos < tiles) {
+        ckey = kDkdvKeys * (tile0 - cpos);
+        cpos = tile0;
+      } else {
+        cpos += tiles;
+        next_segment();
+      }
+    }
+  }
   Half t0 = half_here();
   issue_k(t0, 0);
   issue_ds(t0, 0);
@@ -1171,6 +1253,22 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
   }
   __syncthreads();  // every LDS read is done: the buffers are free for the row staging
   if (!wave_ok) return;
+  if constexpr (kPart) {
+    const int slot = item[PT_SLOT];
+    if (slot >= 0) {  // partial rows, in register order
+      f32x4* p = reinterpret_cast<f32x4*>(a.part_ws + static_cast<int64_t>(slot) * kQSlot) +
+                 wave * 2048 + lane;
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            p[(16 * j + 4 * db + g) * 64] =
+                f32x4{dq[j][db][4 * g], dq[j][db][4 * g + 1], dq[j][db][4 * g + 2], dq[j][db][4 * g + 3]};
+      return;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < 2; j++)
     if (tw0 + 32 * j < len)
@@ -1179,6 +1277,38 @@ __global__ __launch_bounds__(512) void mfma_dqs(KernelArgs a) {
                       qstride, len - tw0 - 32 * j, lane);
 }
 
+// Sum of dQ's key parts, part 0 first (blockIdx.y: wave and 32-query half).
+__global__ __launch_bounds__(256) void mfma_dqs_merge(KernelArgs a) {
+  const int32_t* item = a.plan + a.off_merge + PT_WORDS * blockIdx.x;
+  const int leaf = item[PT_LEAF];
+  const int32_t* cu = a.plan + a.off_cu;
+  const int row0 = cu[leaf], len = cu[leaf + 1] - cu[leaf];
+  const int wave = blockIdx.y >> 1, j = blockIdx.y & 1;
+  const int db = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
+  const int head = item[PT_QH] + wave % a.hpw_dqs;
+  const int t = item[PT_TOK] + kDqsTokens * (wave / a.hpw_dqs) + 32 * j + n;
+  if (t >= len) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * kQSlot) +
+                   wave * 2048 + 1024 * j + 256 * db + lane;
+  f32x4 v[4];
+#pragma unroll
+  for (int g = 0; g < 4; g++) v[g] = p[64 * g];
+  const int parts = item[PT_TILES];
+#pragma unroll 4
+  for (int s = 1; s < parts; s++) {
+    p += kQSlot / 4;
+#pragma unroll
+    for (int g = 0; g < 4; g++) v[g] += p[64 * g];
+  }
+  bf16* out = static_cast<bf16*>(a.dq) + (static_cast<int64_t>(row0 + t) * a.hq + head) * kMfmaD + 32 * db + 4 * h;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    bf16x4 o;
+#pragma unroll
+    for (int b = 0; b < 4; b++) o[b] = static_cast<bf16>(v[g][b] * a.scale);
+    *reinterpret_cast<bf16x4*>(out + 8 * g) = o;
+  }
+}
 #endif  // dQ
 
 #if TPR_MFMA_GROUP & 2
@@ -1751,10 +1881,16 @@ bool strided_rows(const KernelArgs& a) {
 #if TPR_MFMA_GROUP & 1
 template <bool kRunList>
 void launch_fwd_tile(const KernelArgs& a, hipStream_t s) {
-  if (strided_rows(a))
-    hipLaunchKernelGGL((mfma_fwd<kRunList, true>), dim3(a.n_items), dim3(64 * kFwdWaves), 0, s, a);
+  const dim3 block(64 * kFwdWaves);
+  if (a.part_ws && strided_rows(a))
+    hipLaunchKernelGGL((mfma_fwd<kRunList, true, true>), dim3(a.n_part), block, 0, s, a);
+  else if (a.part_ws)
+    hipLaunchKernelGGL((mfma_fwd<kRunList, false, true>), dim3(a.n_part), block, 0, s, a);
+  else if (strided_rows(a))
+    hipLaunchKernelGGL((mfma_fwd<kRunList, true, false>), dim3(a.n_items), block, 0, s, a);
   else
-    hipLaunchKernelGGL((mfma_fwd<kRunList, false>), dim3(a.n_items), dim3(64 * kFwdWaves), 0, s, a);
+    hipLaunchKernelGGL((mfma_fwd<kRunList, false, false>), dim3(a.n_items), block, 0, s, a);
+  if (a.part_ws) hipLaunchKernelGGL(mfma_fwd_merge, dim3(a.n_merge, kFwdWaves), dim3(256), 0, s, a);
 }
 #endif
 
@@ -1824,10 +1960,16 @@ int launch_mfma_dkdv(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s) 
 #if TPR_MFMA_GROUP & 4
 int launch_mfma_dq(const KernelArgs& a, int n_fwd, hipStream_t s) {
   if (n_fwd <= 0) return 0;
-  if (a.ds && strided_rows(a))
-    hipLaunchKernelGGL((mfma_dqs<true>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
+  if (a.ds && a.part_ws) {
+    if (strided_rows(a))
+      hipLaunchKernelGGL((mfma_dqs<true, true>), dim3(a.n_part), dim3(64 * kFwdWaves), 0, s, a);
+    else
+      hipLaunchKernelGGL((mfma_dqs<false, true>), dim3(a.n_part), dim3(64 * kFwdWaves), 0, s, a);
+    hipLaunchKernelGGL(mfma_dqs_merge, dim3(a.n_merge, 2 * kFwdWaves), dim3(256), 0, s, a);
+  } else if (a.ds && strided_rows(a))
+    hipLaunchKernelGGL((mfma_dqs<true, false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
   else if (a.ds)
-    hipLaunchKernelGGL((mfma_dqs<false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
+    hipLaunchKernelGGL((mfma_dqs<false, false>), dim3(n_fwd), dim3(64 * kFwdWaves), 0, s, a);
   else if (a.max_runs > kMfmaRegRuns)
     launch_dq_tile<true>(a, n_fwd, s);
   else

@@ -156,10 +156,12 @@ constexpr float kSlack16 = 8.f;  // lazy-rescale slack in log2 units (as the hea
 // kRunList: key runs read from the plan; kStrided: q, k or v rows wider than
 // packed (the packed instance folds every row stride to a constant).
 // ---------------------------------------------------------------------------
-template <int kD, bool kRunList, bool kStrided>
+// kPart: items over part of their key stream (PF_OFF_FPART), for calls whose
+// query rows alone leave compute units idle.
+template <int kD, bool kRunList, bool kStrided, bool kPart>
 __global__ __launch_bounds__(64 * m16_fwd_waves(kD)) void m16_fwd(KernelArgs a) {
   using T = Geo<kD>;
-  const int32_t* item = a.plan + a.off_fwd + 4 * blockIdx.x;
+  const int32_t* item = kPart ? a.plan + a.off_part + PT_WORDS * blockIdx.x : a.plan + a.off_fwd + 4 * blockIdx.x;
   const int leaf = item[0];
   if (leaf < 0) return;
   const int tok0 = item[1], qh0 = item[2], kvh = item[3];
@@ -197,10 +199,11 @@ __global__ __launch_bounds__(64 * m16_fwd_waves(kD)) void m16_fwd(KernelArgs a) 
   };
 
   const auto seg = load_keys<kRunList>(a, leaf, suffix_keys);
-  const int ntiles = seg.ntiles;
+  const int ntiles = kPart ? item[PT_TILES] : seg.ntiles;
   Cursor cc = cursor_begin(seg);  // the tile being copied
+  if constexpr (kPart) cursor_skip(seg, cc, item[PT_TILE0]);
   TileLoc tl_c = cursor_tile(cc);
-  Cursor mc = cursor_begin(seg);  // the tile being computed
+  Cursor mc = kPart ? cc : cursor_begin(seg);  // the tile being computed
   TileLoc tl = cursor_tile(mc);
   copy_tile<kD, kFW>(kv_src(tl_c, true), kv_rb(tl_c, true), tl_c.len, lds0, wave, lane);
   copy_tile<kD, kFW>(kv_src(tl_c, false), kv_rb(tl_c, false), tl_c.len, lds0 + 2 * T::TB, wave, lane);
@@ -366,6 +369,26 @@ __global__ __launch_bounds__(64 * m16_fwd_waves(kD)) void m16_fwd(KernelArgs a) 
     __syncthreads();
   }
 
+  if constexpr (kPart) {
+    const int slot = item[PT_SLOT];
+    if (slot >= 0) {  // partial rows, in register order, then (m, l)
+      constexpr int kSlot = fpart_slot_floats(PATH_MFMA16, kD), kRowsWg = kM16Waves * kM16Tokens;
+      float* ws = a.part_ws + static_cast<int64_t>(slot) * kSlot;
+#pragma unroll
+      for (int qs = 0; qs < kQS; qs++) {
+        const float lt = xsum16(l[qs]);
+        f32x4* po = reinterpret_cast<f32x4*>(ws) + (wave * kQS + qs) * T::ND * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < T::ND; db++) po[64 * db] = o[qs][db];
+        if (g == 0) {
+          float* st = ws + kRowsWg * kD + 2 * (16 * (wave * kQS + qs) + i16);
+          st[0] = m[qs];
+          st[1] = lt;
+        }
+      }
+      return;
+    }
+  }
   // O^T register r of block db: head dim 16 db + 4 g + r of query l % 16
 #pragma unroll
   for (int qs = 0; qs < kQS; qs++) {
@@ -383,6 +406,52 @@ __global__ __launch_bounds__(64 * m16_fwd_waves(kD)) void m16_fwd(KernelArgs a) 
     }
     if (g == 0) a.lse[static_cast<int64_t>(head) * a.total_q + row0 + t] = m[qs] * a.scale + logf(lt);
   }
+}
+
+// Sum of the forward's key parts, part 0 first: O = sum w_p O_p / sum w_p l_p
+// with w_p = exp(m_p - max m). One 16-query sub-block per workgroup row
+// (blockIdx.y), 64 columns per wave.
+template <int kD>
+__global__ __launch_bounds__(kD) void m16_fwd_merge(KernelArgs a) {
+  constexpr int kFW = m16_fwd_waves(kD), kQS = kFW * 16 == kM16Waves * kM16Tokens ? 1 : 2, ND = kD / 16;
+  constexpr int kSlot = fpart_slot_floats(PATH_MFMA16, kD), kRowsWg = kM16Waves * kM16Tokens;
+  const int32_t* item = a.plan + a.off_merge + PT_WORDS * blockIdx.x;
+  const int leaf = item[PT_LEAF];
+  const int32_t* cu = a.plan + a.off_cu;
+  const int row0 = cu[leaf], len = cu[leaf + 1] - cu[leaf];
+  const int sb = blockIdx.y, wave = sb / kQS, db0 = 4 * (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  const int head = item[PT_QH] + wave % a.hpw;
+  const int t = item[PT_TOK] + 16 * kQS * (wave / a.hpw) + 16 * (sb % kQS) + i16;
+  if (t >= len) return;
+  const int parts = item[PT_TILES];
+  const float* ws = a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * kSlot;
+  const float* st = ws + kRowsWg * kD + 2 * (16 * sb + i16);
+  float m = -INFINITY;
+#pragma unroll 4
+  for (int p = 0; p < parts; p++) m = fmaxf(m, st[p * kSlot]);
+  const float c2 = a.scale * kLog2e;
+  float l = 0.f;
+  f32x4 o[4] = {};
+#pragma unroll 4
+  for (int p = 0; p < parts; p++) {
+    const int64_t at = static_cast<int64_t>(p) * kSlot;
+    const float w = fast_exp2((st[at] - m) * c2);
+    l += w * st[at + 1];
+    const f32x4* po = reinterpret_cast<const f32x4*>(ws + at) + (sb * ND + db0) * 64 + lane;
+#pragma unroll
+    for (int x = 0; x < 4; x++) o[x] += w * po[64 * x];
+  }
+  const float inv = 1.f / l;
+  bf16* out = static_cast<bf16*>(a.out) + (static_cast<int64_t>(row0 + t) * a.hq + head) * kD + 16 * db0 + 4 * g;
+#pragma unroll
+  for (int x = 0; x < 4; x++) {
+    bf16x4 v;
+#pragma unroll
+    for (int b = 0; b < 4; b++) v[b] = static_cast<bf16>(o[x][b] * inv);
+    *reinterpret_cast<bf16x4*>(out + 16 * x) = v;
+  }
+  if (db0 == 0 && g == 0) a.lse[static_cast<int64_t>(head) * a.total_q + row0 + t] = m * a.scale + logf(l);
 }
 
 // ---------------------------------------------------------------------------
@@ -429,16 +498,26 @@ __global__ __launch_bounds__(256) void m16_delta(KernelArgs a) {
   }
 }
 
+// A wave's dQ rows of one key part, in register order.
+template <int kD>
+__device__ __forceinline__ void store_part(float* slot, const f32x4 (&dq)[2][kD / 16], int wave, int lane) {
+  f32x4* p = reinterpret_cast<f32x4*>(slot) + wave * 2 * (kD / 16) * 64 + lane;
+#pragma unroll
+  for (int qs = 0; qs < 2; qs++)
+#pragma unroll
+    for (int db = 0; db < kD / 16; db++) p[(qs * (kD / 16) + db) * 64] = dq[qs][db];
+}
+
 // ---------------------------------------------------------------------------
 // dQ. Same workgroup shape and key stream as the forward. Per 64-key tile:
 // S^T = K Q^T and dP^T = V dO^T (K, V rows from LDS; Q, dO in registers),
 // P = exp2(scale*log2e S - lse*log2e), dS = P (dP - delta), then
 // dQ^T += K^T dS^T with K^T read transposed from the K tile.
 // ---------------------------------------------------------------------------
-template <int kD, bool kRunList, bool kStrided>
+template <int kD, bool kRunList, bool kStrided, bool kPart>  // as m16_fwd
 __global__ __launch_bounds__(256) void m16_dq(KernelArgs a) {
   using T = Geo<kD>;
-  const int32_t* item = a.plan + a.off_fwd + 4 * blockIdx.x;
+  const int32_t* item = kPart ? a.plan + a.off_part + PT_WORDS * blockIdx.x : a.plan + a.off_fwd + 4 * blockIdx.x;
   const int leaf = item[0];
   if (leaf < 0) return;
   const int tok0 = item[1], qh0 = item[2], kvh = item[3];
@@ -472,10 +551,11 @@ __global__ __launch_bounds__(256) void m16_dq(KernelArgs a) {
   };
 
   const auto seg = load_keys<kRunList>(a, leaf, suffix_keys);
-  const int ntiles = seg.ntiles;
+  const int ntiles = kPart ? item[PT_TILES] : seg.ntiles;
   Cursor cc = cursor_begin(seg);
+  if constexpr (kPart) cursor_skip(seg, cc, item[PT_TILE0]);
   TileLoc tl_c = cursor_tile(cc);
-  Cursor mc = cursor_begin(seg);
+  Cursor mc = kPart ? cc : cursor_begin(seg);
   TileLoc tl = cursor_tile(mc);
   copy_tile<kD>(kv_src(tl_c, true), kv_rb(tl_c, true), tl_c.len, lds0, wave, lane);
   copy_tile<kD>(kv_src(tl_c, false), kv_rb(tl_c, false), tl_c.len, lds0 + 2 * T::TB, wave, lane);
@@ -604,6 +684,13 @@ __global__ __launch_bounds__(256) void m16_dq(KernelArgs a) {
     __syncthreads();
   }
 
+  if constexpr (kPart) {
+    if (item[PT_SLOT] >= 0) {
+      store_part<kD>(a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * qpart_slot_floats(PATH_MFMA16, kD, false), dq,
+                     wave, lane);
+      return;
+    }
+  }
 #pragma unroll
   for (int qs = 0; qs < 2; qs++) {
     const int t = tw0 + 16 * qs + i16;
@@ -638,12 +725,12 @@ __global__ __launch_bounds__(256) void m16_dq(KernelArgs a) {
 // (the HBM stream) are copied two tiles ahead of the one being computed into
 // three buffers, the K rows (mostly L2 hits) one tile ahead into two: 160 KiB.
 // ---------------------------------------------------------------------------
-template <int kD, bool kStrided>
+template <int kD, bool kStrided, bool kPart>  // as m16_fwd
 __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
   using T = Geo<kD>;
   static_assert(kD == 256, "the dS store serves head_dim 256 on this family");
   constexpr int kW = kM16DqsWaves;
-  const int32_t* item = a.plan + a.off_dqs + 4 * blockIdx.x;
+  const int32_t* item = kPart ? a.plan + a.off_part + PT_WORDS * blockIdx.x : a.plan + a.off_dqs + 4 * blockIdx.x;
   const int leaf = item[0];
   if (leaf < 0) return;
   const int tok0 = item[1], qh0 = item[2], kvh = item[3];
@@ -732,6 +819,7 @@ __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
     cpos++;
     if (ckey >= clim) next_segment();
   };
+  const int cend = kPart ? item[PT_TILE0] + item[PT_TILES] : 0;  // past the part's last tile
   const char* ds_wave = nullptr;  // this wave's dS blocks: first slot of its query block, its head and half
   if (wave_ok) {
     const int first = plan_word(a.plan + a.off_ds_first + qb);
@@ -753,7 +841,7 @@ __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
   auto tile_here = [&]() __attribute__((always_inline)) {
     const bool suffix = cd == depth;
     Tile t;
-    t.more = clim > 0;
+    t.more = clim > 0 && (!kPart || cpos < cend);
     t.rb = suffix ? k_rb : p_rb;
     t.k = (suffix ? kbase : pkbase) + static_cast<int64_t>(crow + ckey) * t.rb;
     t.rows = min(kKeys, clen - ckey);
@@ -829,6 +917,19 @@ __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
   // outstanding means both K and dS of the next tile have landed.
   static_assert(T::TB / 1024 / kW == 4, "4 K copies per wave per tile");
   next_segment();
+  if constexpr (kPart) {
+    const int tile0 = item[PT_TILE0];
+    while (cpos < tile0 && clim > 0) {
+      const int tiles = (clim + kKeys - 1) / kKeys;
+      if (tile0 - cpos < tiles) {
+        ckey = kKeys * (tile0 - cpos);
+        cpos = tile0;
+      } else {
+        cpos += tiles;
+        next_segment();
+      }
+    }
+  }
   Tile t0 = tile_here();
   issue_k(t0, 0);
   issue_ds(t0, 0);
@@ -856,6 +957,13 @@ __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
   }
 
   if (!wave_ok) return;
+  if constexpr (kPart) {
+    if (item[PT_SLOT] >= 0) {
+      store_part<kD>(a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * qpart_slot_floats(PATH_MFMA16, kD, true), dq,
+                     wave, lane);
+      return;
+    }
+  }
 #pragma unroll
   for (int qs = 0; qs < 2; qs++) {
     const int t = tw0 + 16 * qs + i16;
@@ -868,6 +976,40 @@ __global__ __launch_bounds__(64 * kM16DqsWaves) void m16_dqs(KernelArgs a) {
       for (int r = 0; r < 4; r++) v4[r] = static_cast<bf16>(dq[qs][db][r] * a.scale);
       *reinterpret_cast<bf16x4*>(dp + 16 * db) = v4;
     }
+  }
+}
+
+// Sum of dQ's key parts, part 0 first: a 16-query sub-block per workgroup row
+// (blockIdx.y), 64 columns per wave; hpw query heads per item.
+template <int kD>
+__global__ __launch_bounds__(kD) void m16_dq_merge(KernelArgs a, int hpw, int slot_floats) {
+  const int32_t* item = a.plan + a.off_merge + PT_WORDS * blockIdx.x;
+  const int leaf = item[PT_LEAF];
+  const int32_t* cu = a.plan + a.off_cu;
+  const int row0 = cu[leaf], len = cu[leaf + 1] - cu[leaf];
+  const int sb = blockIdx.y, wave = sb >> 1, db0 = 4 * (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  const int head = item[PT_QH] + wave % hpw, t = item[PT_TOK] + kM16Tokens * (wave / hpw) + 16 * (sb & 1) + i16;
+  if (t >= len) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(a.part_ws + static_cast<int64_t>(item[PT_SLOT]) * slot_floats) +
+                   (sb * (kD / 16) + db0) * 64 + lane;
+  f32x4 v[4];
+#pragma unroll
+  for (int x = 0; x < 4; x++) v[x] = p[64 * x];
+  const int parts = item[PT_TILES];
+#pragma unroll 4
+  for (int s = 1; s < parts; s++) {
+    p += slot_floats / 4;
+#pragma unroll
+    for (int x = 0; x < 4; x++) v[x] += p[64 * x];
+  }
+  bf16* out = static_cast<bf16*>(a.dq) + (static_cast<int64_t>(row0 + t) * a.hq + head) * kD + 16 * db0 + 4 * g;
+#pragma unroll
+  for (int x = 0; x < 4; x++) {
+    bf16x4 o;
+#pragma unroll
+    for (int b = 0; b < 4; b++) o[b] = static_cast<bf16>(v[x][b] * a.scale);
+    *reinterpret_cast<bf16x4*>(out + 16 * x) = o;
   }
 }
 
@@ -1232,10 +1374,17 @@ bool strided_rows(const KernelArgs& a) {
 
 template <int kD, bool kRunList>
 void launch_fwd_runs(const KernelArgs& a, hipStream_t s) {
-  if (strided_rows<kD>(a))
-    hipLaunchKernelGGL((m16_fwd<kD, kRunList, true>), dim3(a.n_items), dim3(64 * m16_fwd_waves(kD)), 0, s, a);
+  const dim3 block(64 * m16_fwd_waves(kD));
+  if (a.part_ws && strided_rows<kD>(a))
+    hipLaunchKernelGGL((m16_fwd<kD, kRunList, true, true>), dim3(a.n_part), block, 0, s, a);
+  else if (a.part_ws)
+    hipLaunchKernelGGL((m16_fwd<kD, kRunList, false, true>), dim3(a.n_part), block, 0, s, a);
+  else if (strided_rows<kD>(a))
+    hipLaunchKernelGGL((m16_fwd<kD, kRunList, true, false>), dim3(a.n_items), block, 0, s, a);
   else
-    hipLaunchKernelGGL((m16_fwd<kD, kRunList, false>), dim3(a.n_items), dim3(64 * m16_fwd_waves(kD)), 0, s, a);
+    hipLaunchKernelGGL((m16_fwd<kD, kRunList, false, false>), dim3(a.n_items), block, 0, s, a);
+  if (a.part_ws)
+    hipLaunchKernelGGL(m16_fwd_merge<kD>, dim3(a.n_merge, kM16Waves * kM16Tokens / 16), dim3(kD), 0, s, a);
 }
 
 template <int kD>
@@ -1272,20 +1421,36 @@ int launch_dkdv_d(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s) {
 
 template <int kD, bool kRunList>
 void launch_dq_runs(const KernelArgs& a, int n_fwd, hipStream_t s) {
-  if (strided_rows<kD>(a))
-    hipLaunchKernelGGL((m16_dq<kD, kRunList, true>), dim3(n_fwd), dim3(64 * kM16Waves), 0, s, a);
+  const dim3 block(64 * kM16Waves);
+  if (a.part_ws && strided_rows<kD>(a))
+    hipLaunchKernelGGL((m16_dq<kD, kRunList, true, true>), dim3(a.n_part), block, 0, s, a);
+  else if (a.part_ws)
+    hipLaunchKernelGGL((m16_dq<kD, kRunList, false, true>), dim3(a.n_part), block, 0, s, a);
+  else if (strided_rows<kD>(a))
+    hipLaunchKernelGGL((m16_dq<kD, kRunList, true, false>), dim3(n_fwd), block, 0, s, a);
   else
-    hipLaunchKernelGGL((m16_dq<kD, kRunList, false>), dim3(n_fwd), dim3(64 * kM16Waves), 0, s, a);
+    hipLaunchKernelGGL((m16_dq<kD, kRunList, false, false>), dim3(n_fwd), block, 0, s, a);
+  if (a.part_ws)
+    hipLaunchKernelGGL(m16_dq_merge<kD>, dim3(a.n_merge, 2 * kM16Waves), dim3(kD), 0, s, a, a.hpw,
+                       qpart_slot_floats(PATH_MFMA16, kD, false));
 }
 
 template <int kD>
 int launch_dq_d(const KernelArgs& a, int n_fwd, hipStream_t s) {
   if constexpr (kD == 256) {
     if (n_fwd > 0 && a.ds) {  // dQ from the dS store
-      if (strided_rows<kD>(a))
-        hipLaunchKernelGGL((m16_dqs<kD, true>), dim3(n_fwd), dim3(64 * kM16DqsWaves), 0, s, a);
+      const dim3 block(64 * kM16DqsWaves);
+      if (a.part_ws && strided_rows<kD>(a))
+        hipLaunchKernelGGL((m16_dqs<kD, true, true>), dim3(a.n_part), block, 0, s, a);
+      else if (a.part_ws)
+        hipLaunchKernelGGL((m16_dqs<kD, false, true>), dim3(a.n_part), block, 0, s, a);
+      else if (strided_rows<kD>(a))
+        hipLaunchKernelGGL((m16_dqs<kD, true, false>), dim3(n_fwd), block, 0, s, a);
       else
-        hipLaunchKernelGGL((m16_dqs<kD, false>), dim3(n_fwd), dim3(64 * kM16DqsWaves), 0, s, a);
+        hipLaunchKernelGGL((m16_dqs<kD, false, false>), dim3(n_fwd), block, 0, s, a);
+      if (a.part_ws)
+        hipLaunchKernelGGL(m16_dq_merge<kD>, dim3(a.n_merge, 2 * kM16DqsWaves), dim3(kD), 0, s, a, a.hpw_dqs,
+                           qpart_slot_floats(PATH_MFMA16, kD, true));
       return hipGetLastError() != hipSuccess ? 4 : 0;
     }
   }

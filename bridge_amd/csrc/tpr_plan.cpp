@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <functional>
 #include <numeric>
 #include <vector>
 
@@ -86,6 +87,119 @@ std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words
     out.clear();
     *count = 0;
   }
+  return out;
+}
+
+// ---- key parts ----------------------------------------------------------------
+// A forward / dQ item is one workgroup, and a compute unit holds one: with few
+// items (or a last round of few) most units idle while the longest streams
+// run. Such a list is cut along the keys into parts of at most `limit` tiles;
+// the limit is the one with the least estimated time, or none.
+struct QueryItem {
+  int32_t leaf, tok, qh, kvh, tiles;
+};
+
+// Makespan, in tiles, of work of the given costs (sorted, longest first) dealt
+// as order_for_xcds deals it: each to its KV head's XCDs, there to the first
+// free slot (per_cu workgroups share a compute unit).
+int list_makespan(const std::vector<std::pair<int, int>>& work, int hkv, int per_cu) {  // (cost, KV head)
+  const int slots = kPlanCus / kXcds * per_cu;
+  std::vector<int> ends(static_cast<size_t>(kXcds) * slots, 0);  // min-heap of end times per XCD
+  int64_t load[kXcds] = {};
+  int count[kXcds] = {}, end = 0;
+  for (const auto& w : work) {
+    int best = -1;
+    if (hkv % kXcds == 0) {
+      best = w.second % kXcds;
+    } else {
+      const bool own = kXcds % hkv == 0;
+      for (int x = own ? w.second : 0; x < kXcds; x += own ? hkv : 1)
+        if (best < 0 || load[x] < load[best]) best = x;
+    }
+    load[best] += w.first;
+    int* heap = &ends[static_cast<size_t>(best) * slots];
+    if (count[best] < slots) {  // a slot not used yet (costs only fall, so no heap order is needed before)
+      heap[count[best]++] = w.first;
+      end = std::max(end, w.first);
+      if (count[best] == slots) std::make_heap(heap, heap + slots, std::greater<int>());
+    } else {
+      std::pop_heap(heap, heap + slots, std::greater<int>());
+      heap[slots - 1] += w.first;
+      end = std::max(end, heap[slots - 1]);
+      std::push_heap(heap, heap + slots, std::greater<int>());
+    }
+  }
+  return end;
+}
+
+struct Parts {
+  std::vector<int32_t> items, merges;
+  int32_t n_items = 0, n_merges = 0, slots = 0;
+};
+
+// `fixed`: a workgroup's start and end; `merge`: the second launch; `per_slot`:
+// writing and reading one partial slot, over all units -- all in tiles (1.2 us
+// for the forward at head_dim 128; 0.084 us a slot there). Fixed numbers of
+// parts against the limit chosen here, forward us at GQA 32/8, d128 (1, 2, 4,
+// 8, 16 parts; chosen): prefix 8192 + 512: 163, 97, 80, 94, 118; 80. 32768 +
+// 40: 590, 303, 159, 88, 60; 57. 4096 + 1000: 103, 86, 95, 120, 183; 85.
+// 4096 + 2048: 159, 175, 199, 261, 385; 160 (not cut). d64, 8192 + 512: 136,
+// 80, 62, 63, 69; 59. d256, GQA 8/2: 242, 130, 77, 57, 71; 57.
+Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double fixed, double merge, double per_slot) {
+  Parts out;
+  constexpr int kLeastTiles = 3;
+  const size_t units = static_cast<size_t>(kPlanCus) * per_cu;
+  if (list.empty() || list.size() >= 4 * units) return out;
+  int longest = 0;
+  for (const QueryItem& q : list) longest = std::max(longest, q.tiles);
+  std::vector<std::pair<int, int>> work;
+  auto estimate = [&](int limit) {
+    work.clear();
+    int slots = 0;
+    for (const QueryItem& q : list) {
+      const int n = (q.tiles + limit - 1) / limit;
+      for (int p = 0; p < n; p++)
+        work.emplace_back(q.tiles * (p + 1) / n - q.tiles * p / n + static_cast<int>(fixed), q.kvh);
+      if (n > 1) slots += n;
+    }
+    std::sort(work.begin(), work.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
+    return list_makespan(work, hkv, per_cu) + (slots ? merge + per_slot * slots : 0.0);
+  };
+  const double whole = estimate(longest);
+  // less than this is not worth a second launch: a full chip, or short streams
+  int64_t total = 0;
+  for (const auto& w : work) total += w.first;
+  double best = 0.92 * whole;
+  if (static_cast<double>(total) / units + merge >= best) return out;
+  int limit = 0;
+  for (int cut : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+    const int l = (longest + cut - 1) / cut;
+    // parts over two rounds of the chip only add slots
+    if (l < kLeastTiles || (cut > 2 && work.size() > 2 * units)) break;
+    const double e = estimate(l);
+    if (e < best) {
+      best = e;
+      limit = l;
+    }
+  }
+  if (limit == 0) return out;
+  std::vector<Item> items;
+  for (const QueryItem& q : list) {
+    const int n = (q.tiles + limit - 1) / limit;
+    if (n > 1) {
+      out.merges.insert(out.merges.end(), {q.leaf, q.tok, q.qh, q.kvh, 0, n, out.slots, 0});
+      out.n_merges++;
+    }
+    for (int p = 0; p < n; p++) {
+      const int t0 = q.tiles * p / n, t1 = q.tiles * (p + 1) / n;
+      Item it;
+      it.words = {q.leaf, q.tok, q.qh, q.kvh, t0, t1 - t0, n > 1 ? out.slots++ : -1, 0};
+      it.work = t1 - t0;
+      it.kvh = q.kvh;
+      items.push_back(std::move(it));
+    }
+  }
+  out.items = order_for_xcds(items, hkv, PT_WORDS, &out.n_items);
   return out;
 }
 
@@ -430,6 +544,36 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
     dqs_words = query_items(heads, tokens, &n_dqs);
   }
 
+  // ---- key parts of the forward and of dQ from the store --------------------------
+  // tiles of an item's key stream: its node (or merged run) and suffix pieces
+  Parts fparts, qparts;
+  if (mfma_family) {
+    std::vector<QueryItem> fwd_list, dqs_list;
+    auto suffix_tiles = [&](const int32_t* w, int tokens, int keys) {
+      return (std::min(cu[w[0] + 1] - cu[w[0]], w[1] + tokens) + keys - 1) / keys;
+    };
+    for (int i = 0; i < n_fwd; i++) {
+      const int32_t* w = &fwd_words[4 * i];
+      if (w[0] < 0) continue;
+      int tiles = suffix_tiles(w, tokens_per_wg, kFwdKeys);
+      for (size_t r = 1; r < leaf_runs[w[0]].size(); r += 2) tiles += (leaf_runs[w[0]][r] + kFwdKeys - 1) / kFwdKeys;
+      fwd_list.push_back({w[0], w[1], w[2], w[3], tiles});
+    }
+    const int fwd_per_cu = D == 64 ? 3 : 1, dq_per_cu = D == 64 ? 2 : 1;
+    const double slot = D == 128 ? 0.07 : 0.035;
+    fparts = key_parts(fwd_list, Hkv, fwd_per_cu, 4, 4, slot);
+    if (n_dqs > 0) {
+      const int tokens = (path == PATH_MFMA ? kDqsTokens : kM16Tokens) * (kM16DqsWaves / gcd_int(G, kM16DqsWaves));
+      for (int i = 0; i < n_dqs; i++) {
+        const int32_t* w = &dqs_words[4 * i];
+        if (w[0] >= 0) dqs_list.push_back({w[0], w[1], w[2], w[3], ds_table[M + w[0]] + suffix_tiles(w, tokens, KT)});
+      }
+      qparts = key_parts(dqs_list, Hkv, 1, 3, 2, 0.07);
+    } else if (path == PATH_MFMA16) {
+      qparts = key_parts(fwd_list, Hkv, dq_per_cu, 4, 4, slot);
+    }
+  }
+
   // ---- assemble ----------------------------------------------------------------
   plan.assign(PF_HEADER_WORDS, 0);
   auto append = [&](const int32_t* src, size_t count) {
@@ -472,6 +616,15 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   plan[PF_OFF_DS] = ds_table.empty() ? 0 : append(ds_table.data(), ds_table.size());
   plan[PF_MASK_COLS] = static_cast<int32_t>(mask_cols);
   plan[PF_SPLIT] = split;
+  auto append_parts = [&](const Parts& p, int n_item, int off_item, int n_merge, int off_merge, int slots) {
+    plan[n_item] = p.n_items;
+    plan[off_item] = append(p.items.data(), p.items.size());
+    plan[n_merge] = p.n_merges;
+    plan[off_merge] = append(p.merges.data(), p.merges.size());
+    plan[slots] = p.slots;
+  };
+  append_parts(fparts, PF_N_FPART, PF_OFF_FPART, PF_N_FMERGE, PF_OFF_FMERGE, PF_FSLOTS);
+  append_parts(qparts, PF_N_QPART, PF_OFF_QPART, PF_N_QMERGE, PF_OFF_QMERGE, PF_QSLOTS);
   plan[PF_N_DQS] = n_dqs;
   plan[PF_OFF_DQS] = dqs_words.empty() ? 0 : append(dqs_words.data(), dqs_words.size());
   plan[PF_TOTAL_WORDS] = static_cast<int32_t>(plan.size());

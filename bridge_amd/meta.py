@@ -57,7 +57,8 @@ class LaunchPlan:
 
     host: torch.Tensor     # int32, CPU
     device: torch.Tensor   # int32, on the compute device
-    workspace_bytes: int
+    workspace_bytes: int          # backward
+    fwd_workspace_bytes: int = 0  # forward key parts (few query rows), else 0
 
     @property
     def path(self) -> str:
@@ -266,16 +267,23 @@ class TPRPrefixMeta:
                                 code, flags, ctypes.cast(cu, ctypes.c_void_p), ctypes.cast(no, ctypes.c_void_p),
                                 ctypes.cast(an, ctypes.c_void_p),
                                 _lib.TPR_DS_STORE_DEFAULT if budget is None else budget)
+        # one call builds and copies the plan unless it outgrows the guess (a
+        # second call would build it again)
         words = ctypes.c_int64(0)
-        _lib.check(lib.tpr_attn_plan(ctypes.byref(desc), None, 0, ctypes.byref(words)), "tpr_attn_plan")
-        host = torch.empty(int(words.value), dtype=torch.int32)
-        _lib.check(lib.tpr_attn_plan(ctypes.byref(desc), ctypes.c_void_p(host.data_ptr()), host.numel(),
-                                     ctypes.byref(words)), "tpr_attn_plan")
+        host = torch.empty(1 << 18, dtype=torch.int32)
+        status = lib.tpr_attn_plan(ctypes.byref(desc), ctypes.c_void_p(host.data_ptr()), host.numel(),
+                                   ctypes.byref(words))
+        if status == _lib.TPR_ERR_BUFFER_TOO_SMALL:
+            host = torch.empty(int(words.value), dtype=torch.int32)
+            status = lib.tpr_attn_plan(ctypes.byref(desc), ctypes.c_void_p(host.data_ptr()), host.numel(),
+                                       ctypes.byref(words))
+        _lib.check(status, "tpr_attn_plan")
+        host = host[:int(words.value)].clone()
         if device.type == "cpu":
             dev = host
         else:
             dev = host.to(device, non_blocking=False)
         ws = int(lib.tpr_attn_bwd_workspace_bytes(ctypes.c_void_p(host.data_ptr())))
-        plan = LaunchPlan(host, dev, ws)
+        plan = LaunchPlan(host, dev, ws, int(lib.tpr_attn_fwd_workspace_bytes(ctypes.c_void_p(host.data_ptr()))))
         self._plans[key] = plan
         return plan

@@ -175,7 +175,14 @@ def _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask=None):
         plan.host.data_ptr(), plan.device.data_ptr(),
         _ptr(q), _ptr(k), _ptr(v), _ptr(prefix_k), _ptr(prefix_v), _ptr(out), _ptr(lse),
         _row_stride(q), _row_stride(k), _row_stride(v), *_mask_args(mask))
-    _lib.check(lib.tpr_attn_fwd(ctypes.byref(params), ctypes.c_void_p(_stream_handle(q.device))), "tpr_attn_fwd")
+    ws = None
+    if plan.fwd_workspace_bytes:
+        try:
+            ws = torch.empty(plan.fwd_workspace_bytes, dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            pass  # the forward runs without key parts
+    _lib.check(lib.tpr_attn_fwd_ws(ctypes.byref(params), _ptr(ws), plan.fwd_workspace_bytes,
+                                   ctypes.c_void_p(_stream_handle(q.device))), "tpr_attn_fwd")
     return out, lse
 
 

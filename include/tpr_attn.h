@@ -227,6 +227,18 @@ size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host);
 /* Enqueue the forward on `stream` (a hipStream_t; NULL = default stream). */
 int tpr_attn_fwd(const TprFwdParams* params, void* stream);
 
+/* The forward with a workspace. A plan whose query rows are too few for the
+ * chip may cut its key streams into parts, which leave fp32 partial rows in a
+ * caller-provided workspace (256-byte aligned, at least
+ * tpr_attn_fwd_workspace_bytes() bytes, free again when the call's work on
+ * the stream is done) and are summed in a fixed order. workspace == NULL, or a
+ * plan that needs none: the same as tpr_attn_fwd. Results agree within
+ * rounding (the sums' order differs). */
+int tpr_attn_fwd_ws(const TprFwdParams* params, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace tpr_attn_fwd_ws uses for this plan (0: none). */
+size_t tpr_attn_fwd_workspace_bytes(const int32_t* plan_host);
+
 /* Enqueue the backward on `stream` (all phases, in order). */
 int tpr_attn_bwd(const TprBwdParams* params, void* stream);
 
