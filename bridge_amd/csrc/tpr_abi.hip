@@ -1,6 +1,7 @@
 // tpr_abi.hip -- extern "C" entry points of libtpr_attn.so: argument checks,
 // plan-header decoding and kernel dispatch. Host code only.
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -220,13 +221,16 @@ size_t stat_floats(const int32_t* ph) {
 
 namespace tpr {
 namespace {
+// an fp32 partial slot of dK/dV: a key tile's dK, then its dV
+size_t dkdv_slot_bytes(const int32_t* ph) {
+  const size_t keys = ph[PF_PATH] == PATH_MFMA16 ? m16_keys(ph[PF_D]) : kDkdvKeys;
+  return keys * static_cast<size_t>(ph[PF_D]) * 2 * sizeof(float);
+}
 // bytes before the dS store: the stat area and the fp32 partial slots
 // (a multiple of 256: the stat rows are padded to 64 floats, a slot is
 // keys x D x 2 floats)
 size_t ws_fp32_bytes(const int32_t* ph) {
-  const size_t slots = static_cast<size_t>(ph[PF_N_SLOTS]);
-  const size_t keys = ph[PF_PATH] == PATH_MFMA16 ? m16_keys(ph[PF_D]) : kDkdvKeys;  // per partial slot
-  return (stat_floats(ph) + slots * keys * static_cast<size_t>(ph[PF_D]) * 2) * sizeof(float);
+  return stat_floats(ph) * sizeof(float) + static_cast<size_t>(ph[PF_N_SLOTS]) * dkdv_slot_bytes(ph);
 }
 size_t ds_bytes(const int32_t* ph) {
   return static_cast<size_t>(ph[PF_DS_SLOTS]) * static_cast<size_t>(ph[PF_HQ]) * ds_head_bytes(ph[PF_PATH], ph[PF_D]);
@@ -236,11 +240,13 @@ size_t ds_bytes(const int32_t* ph) {
 
 namespace tpr {
 namespace {
-// the workspace the backward cannot run without; dQ's key parts follow it
+// the workspace the backward cannot run without; dQ's key parts and the dK/dV
+// parts' slots follow it
 size_t bwd_base_bytes(const int32_t* ph) { return ws_fp32_bytes(ph) + ds_bytes(ph); }
 size_t qpart_bytes(const int32_t* ph) {
   return static_cast<size_t>(ph[PF_QSLOTS]) * qpart_slot_floats(ph[PF_PATH], ph[PF_D], ph[PF_DS_SLOTS] > 0) * sizeof(float);
 }
+size_t kpart_bytes(const int32_t* ph) { return static_cast<size_t>(ph[PF_KSLOTS]) * dkdv_slot_bytes(ph); }
 size_t fpart_bytes(const int32_t* ph) {
   return static_cast<size_t>(ph[PF_FSLOTS]) * fpart_slot_floats(ph[PF_PATH], ph[PF_D]) * sizeof(float);
 }
@@ -250,6 +256,11 @@ size_t fpart_bytes(const int32_t* ph) {
 extern "C" size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host) {
   if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
   return bwd_base_bytes(plan_host) + qpart_bytes(plan_host);
+}
+
+extern "C" size_t tpr_attn_bwd_parts_workspace_bytes(const int32_t* plan_host) {
+  if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
+  return bwd_base_bytes(plan_host) + qpart_bytes(plan_host) + kpart_bytes(plan_host);
 }
 
 extern "C" size_t tpr_attn_fwd_workspace_bytes(const int32_t* plan_host) {
@@ -342,7 +353,7 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
       (rc = check_tensor(p->dprefix_k, "dprefix_k", any_p, mfma)) ||
       (rc = check_tensor(p->dprefix_v, "dprefix_v", any_p, mfma)))
     return rc;
-  // dQ runs in key parts where the workspace holds them too (the
+  // dQ and dK/dV run in parts where the workspace holds them too (the
   // allocation-free backward's scratch may not)
   const size_t need = bwd_base_bytes(ph);
   if (need > 0 && (!workspace || workspace_bytes < need))
@@ -384,10 +395,17 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
     a.off_merge = ph[PF_OFF_QMERGE];
     a.n_merge = ph[PF_N_QMERGE];
   }
+  const bool kparts = ph[PF_N_KPART] > 0 && workspace_bytes >= need + qpart_bytes(ph) + kpart_bytes(ph);
+  if (kparts) {
+    a.off_dkdv = ph[PF_OFF_KPART];
+    a.off_red = ph[PF_OFF_KRED];
+    a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + need + qpart_bytes(ph));
+  }
   const bool fp32 = ph[PF_DTYPE] == TPR_DTYPE_FP32;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int n_dkdv = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) ? ph[PF_N_DKDV] : 0;
-  const int n_red = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[PF_N_RED] : 0;  // 0 on the general path
+  const int n_dkdv = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) ? ph[kparts ? PF_N_KPART : PF_N_DKDV] : 0;
+  // 0 on the general path
+  const int n_red = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[kparts ? PF_N_KRED : PF_N_RED] : 0;
   // dQ work items: the forward's, or a dS-store plan's own list
   const int n_dq = (phases & TPR_BWD_DQ) ? (ph[PF_N_DQS] > 0 ? ph[PF_N_DQS] : ph[PF_N_FWD]) : 0;
   if (phases & TPR_BWD_DELTA)
@@ -472,5 +490,8 @@ extern "C" int tpr_attn_bwd_noalloc(const TprBwdParams* p, void* stream) {
   void* ws = nullptr;
   int rc = scratch_for_current_device(static_cast<hipStream_t>(stream), &ws);
   if (rc) return rc;
-  return bwd_phases(p, TPR_BWD_DELTA | TPR_BWD_DKDV | TPR_BWD_DQ, stream, ws, kScratchBytes);
+  // as tpr_attn_bwd with that many bytes runs: whole dK/dV items, and dQ's key
+  // parts where the scratch holds them
+  const size_t bytes = std::min(kScratchBytes, tpr_attn_bwd_workspace_bytes(p->plan_host));
+  return bwd_phases(p, TPR_BWD_DELTA | TPR_BWD_DKDV | TPR_BWD_DQ, stream, ws, bytes);
 }

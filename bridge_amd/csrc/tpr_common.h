@@ -9,7 +9,7 @@
 namespace tpr {
 
 constexpr int32_t kPlanMagic = 0x31525054;  // "TPR1"
-constexpr int32_t kPlanVersion = 8;
+constexpr int32_t kPlanVersion = 9;
 
 // Header word indices.
 enum PlanField : int {
@@ -70,7 +70,15 @@ enum PlanField : int {
   PF_N_QMERGE,
   PF_OFF_QMERGE,
   PF_QSLOTS,
-  PF_HEADER_WORDS = 48
+  // dK/dV parts: the dK/dV items with their query ranges cut finer (no pairs),
+  // the reduction items of their partial slots, and those slots, which follow
+  // dQ's in the caller's workspace (0 items: the lists above)
+  PF_N_KPART,
+  PF_OFF_KPART,
+  PF_N_KRED,
+  PF_OFF_KRED,
+  PF_KSLOTS,
+  PF_HEADER_WORDS = 56
 };
 
 enum KernelPath : int32_t {
@@ -144,6 +152,7 @@ constexpr int kDkdvQ = 64;            // queries per staged query block
 constexpr int kDkdvMaxBlocks = 256;   // query blocks one dK/dV item may stream (LDS table size)
 constexpr int kDkdvPrefixChunk = 64;  // smallest chunk a prefix tile is split into
 constexpr int kPlanCus = 256;         // compute units the dK/dV work is balanced over (MI355X)
+constexpr int kRedSplit = 8;          // workgroups per reduction item: one each left the chip idle
 // dS store (bf16 head_dim 128 and 256): the dK/dV kernel writes each dS block
 // it computes, bf16, and dQ = scale dS K reads them instead of recomputing S
 // and dP. One slot per (dK/dV key tile, query block it is visible to) holds,

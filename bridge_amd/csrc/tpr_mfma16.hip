@@ -1345,12 +1345,13 @@ __global__ __launch_bounds__(256) void m16_reduce(KernelArgs a) {
   bf16* dkd = static_cast<bf16*>(prefix ? a.dpk : a.dk);
   bf16* dvd = static_cast<bf16*>(prefix ? a.dpv : a.dv);
   const int64_t slot_floats = 2 * kKeys * kD;
-  for (int e = threadIdx.x; e < 2 * keys * (kD / 4); e += blockDim.x) {
+  for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < 2 * keys * (kD / 4); e += gridDim.y * blockDim.x) {
     const int which = e / (keys * (kD / 4));  // 0 = dK, 1 = dV
     const int rem = e % (keys * (kD / 4));
     const int key = rem / (kD / 4), d4 = rem % (kD / 4);
     const float* src = a.ws + static_cast<int64_t>(slot0) * slot_floats + which * kKeys * kD + key * kD + 4 * d4;
     f32x4 acc = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
     for (int j = 1; j < nslots; j++) acc += *reinterpret_cast<const f32x4*>(src + j * slot_floats);
     const int64_t at = static_cast<int64_t>(seg_row0 + key0 + key) * kstride + kvh * kD + 4 * d4;
     if (prefix && a.acc_prefix) {
@@ -1413,7 +1414,7 @@ int launch_dkdv_d(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s) {
     if (hipGetLastError() != hipSuccess) return 4;
   }
   if (n_red > 0) {
-    hipLaunchKernelGGL((m16_reduce<kD>), dim3(n_red), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((m16_reduce<kD>), dim3(n_red, kRedSplit), dim3(256), 0, s, a);
     if (hipGetLastError() != hipSuccess) return 4;
   }
   return 0;

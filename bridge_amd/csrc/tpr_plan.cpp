@@ -30,7 +30,7 @@ constexpr int kXcds = 8;
 constexpr int kGenSplitBlocks = 4 * kPlanCus;
 
 struct Item {
-  std::vector<int32_t> words;
+  int32_t words[8];
   int64_t work;
   int32_t kvh;
 };
@@ -73,11 +73,10 @@ std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words
   for (size_t i = 0; i < depth; i++) {
     for (int x = 0; x < kXcds; x++) {
       if (i < queue[x].size()) {
-        out.insert(out.end(), queue[x][i]->words.begin(), queue[x][i]->words.end());
+        out.insert(out.end(), queue[x][i]->words, queue[x][i]->words + words_per_item);
       } else {
-        std::vector<int32_t> empty(words_per_item, 0);
-        empty[0] = -1;
-        out.insert(out.end(), empty.begin(), empty.end());
+        out.push_back(-1);
+        out.insert(out.end(), words_per_item - 1, 0);
       }
     }
   }
@@ -99,36 +98,30 @@ struct QueryItem {
   int32_t leaf, tok, qh, kvh, tiles;
 };
 
-// Makespan, in tiles, of work of the given costs (sorted, longest first) dealt
-// as order_for_xcds deals it: each to its KV head's XCDs, there to the first
-// free slot (per_cu workgroups share a compute unit).
-int list_makespan(const std::vector<std::pair<int, int>>& work, int hkv, int per_cu) {  // (cost, KV head)
-  const int slots = kPlanCus / kXcds * per_cu;
-  std::vector<int> ends(static_cast<size_t>(kXcds) * slots, 0);  // min-heap of end times per XCD
-  int64_t load[kXcds] = {};
-  int count[kXcds] = {}, end = 0;
-  for (const auto& w : work) {
-    int best = -1;
-    if (hkv % kXcds == 0) {
-      best = w.second % kXcds;
-    } else {
-      const bool own = kXcds % hkv == 0;
-      for (int x = own ? w.second : 0; x < kXcds; x += own ? hkv : 1)
-        if (best < 0 || load[x] < load[best]) best = x;
+// Time of one head's workgroup costs (any order) dealt longest first to the
+// first free slot of the XCDs that run that head; every KV head has the same
+// tiles, so one head (or all, where heads share XCDs) stands for the launch.
+int64_t pool_makespan(std::vector<int>& costs, int hkv, int per_cu) {
+  const int copies = hkv % kXcds == 0 ? hkv / kXcds : kXcds % hkv == 0 ? 1 : hkv;
+  const int xcds = hkv % kXcds == 0 ? 1 : kXcds % hkv == 0 ? kXcds / hkv : kXcds;
+  const size_t slots = static_cast<size_t>(xcds) * (kPlanCus / kXcds) * per_cu;
+  std::sort(costs.begin(), costs.end(), std::greater<int>());
+  std::vector<int64_t> ends;
+  ends.reserve(slots);
+  int64_t end = 0;
+  for (int c : costs)
+    for (int i = 0; i < copies; i++) {
+      if (ends.size() < slots) {
+        ends.push_back(c);
+        if (ends.size() == slots) std::make_heap(ends.begin(), ends.end(), std::greater<int64_t>());
+        end = std::max<int64_t>(end, c);
+      } else {
+        std::pop_heap(ends.begin(), ends.end(), std::greater<int64_t>());
+        ends.back() += c;
+        end = std::max(end, ends.back());
+        std::push_heap(ends.begin(), ends.end(), std::greater<int64_t>());
+      }
     }
-    load[best] += w.first;
-    int* heap = &ends[static_cast<size_t>(best) * slots];
-    if (count[best] < slots) {  // a slot not used yet (costs only fall, so no heap order is needed before)
-      heap[count[best]++] = w.first;
-      end = std::max(end, w.first);
-      if (count[best] == slots) std::make_heap(heap, heap + slots, std::greater<int>());
-    } else {
-      std::pop_heap(heap, heap + slots, std::greater<int>());
-      heap[slots - 1] += w.first;
-      end = std::max(end, heap[slots - 1]);
-      std::push_heap(heap, heap + slots, std::greater<int>());
-    }
-  }
   return end;
 }
 
@@ -152,30 +145,30 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
   if (list.empty() || list.size() >= 4 * units) return out;
   int longest = 0;
   for (const QueryItem& q : list) longest = std::max(longest, q.tiles);
-  std::vector<std::pair<int, int>> work;
+  std::vector<int> work;  // one KV head's
   auto estimate = [&](int limit) {
     work.clear();
     int slots = 0;
     for (const QueryItem& q : list) {
+      if (q.kvh != 0) continue;
       const int n = (q.tiles + limit - 1) / limit;
       for (int p = 0; p < n; p++)
-        work.emplace_back(q.tiles * (p + 1) / n - q.tiles * p / n + static_cast<int>(fixed), q.kvh);
+        work.push_back(q.tiles * (p + 1) / n - q.tiles * p / n + static_cast<int>(fixed));
       if (n > 1) slots += n;
     }
-    std::sort(work.begin(), work.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
-    return list_makespan(work, hkv, per_cu) + (slots ? merge + per_slot * slots : 0.0);
+    return static_cast<double>(pool_makespan(work, hkv, per_cu)) + (slots ? merge + per_slot * slots * hkv : 0.0);
   };
   const double whole = estimate(longest);
   // less than this is not worth a second launch: a full chip, or short streams
   int64_t total = 0;
-  for (const auto& w : work) total += w.first;
+  for (int w : work) total += static_cast<int64_t>(w) * hkv;
   double best = 0.92 * whole;
   if (static_cast<double>(total) / units + merge >= best) return out;
   int limit = 0;
   for (int cut : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
     const int l = (longest + cut - 1) / cut;
     // parts over two rounds of the chip only add slots
-    if (l < kLeastTiles || (cut > 2 && work.size() > 2 * units)) break;
+    if (l < kLeastTiles || (cut > 2 && work.size() * hkv > 2 * units)) break;
     const double e = estimate(l);
     if (e < best) {
       best = e;
@@ -192,14 +185,102 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
     }
     for (int p = 0; p < n; p++) {
       const int t0 = q.tiles * p / n, t1 = q.tiles * (p + 1) / n;
-      Item it;
-      it.words = {q.leaf, q.tok, q.qh, q.kvh, t0, t1 - t0, n > 1 ? out.slots++ : -1, 0};
-      it.work = t1 - t0;
-      it.kvh = q.kvh;
-      items.push_back(std::move(it));
+      items.push_back({{q.leaf, q.tok, q.qh, q.kvh, t0, t1 - t0, n > 1 ? out.slots++ : -1, 0}, t1 - t0, q.kvh});
     }
   }
   out.items = order_for_xcds(items, hkv, PT_WORDS, &out.n_items);
+  return out;
+}
+
+// ---- dK/dV parts ----------------------------------------------------------------
+// A dK/dV tile streams every query block that sees it, so with few key tiles,
+// or tiles of unequal ranges, most compute units idle while the longest streams
+// run (prefix 738 + 3016 + 905, GQA 16/2: 54 items, 14 % of the chip busy). The
+// query ranges are then cut into parts of at most `cap` blocks, one cap for
+// node tiles and one for suffix tiles (which then run unpaired), whose fp32
+// partial tiles the reduction pass sums in query-block order.
+struct DkTile {
+  int32_t src, seg, k0, lo, hi;
+};
+int dk_pieces(const DkTile& t, int cap) { return std::max(1, (t.hi - t.lo + cap - 1) / cap); }
+
+// Costs in half head-blocks (64 queries of one head against one key tile; 1.0
+// us at head_dim 128, 1.4 at 256, 0.9 at 64): `fixed` a workgroup's start and
+// end, `pass` the reduction launch, `per_slot` writing and reading a partial.
+Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base, int32_t base_slots, int hkv, int group,
+                 int per_cu, int fixed, double pass, double per_slot) {
+  Parts out;
+  const int units = kPlanCus * per_cu;
+  std::vector<int> costs;
+  int64_t total = 0;
+  for (const Item& it : base)
+    if (it.kvh == 0) {
+      const bool pair = it.words[DK_PAIR] > 0;
+      costs.push_back(static_cast<int>(std::min<int64_t>(2 * (it.work - (pair ? 2 : 1)), 1 << 28)) + fixed + (pair ? fixed / 2 : 0));
+      total += costs.back();
+    }
+  if (costs.empty()) return out;
+  double best = 0.92 * (static_cast<double>(pool_makespan(costs, hkv, per_cu)) + (base_slots ? pass + per_slot * base_slots : 0.0));
+  // a launch this well balanced already is not worth more partials
+  if (static_cast<double>(total) * hkv / units >= best) return out;
+  int longest[2] = {1, 1};
+  for (const DkTile& t : tiles) longest[t.src] = std::max(longest[t.src], t.hi - t.lo);
+  int64_t pieces = 0, slots = 0;
+  auto estimate = [&](int node_cap, int suffix_cap) {
+    costs.clear();
+    pieces = slots = 0;
+    for (const DkTile& t : tiles) {
+      const int n = dk_pieces(t, t.src == 0 ? node_cap : suffix_cap), range = t.hi - t.lo, chunk = (range + n - 1) / n;
+      pieces += n;
+      if (n > 1) slots += n;
+      int left = range;
+      for (int i = 0; i < n; i++, left -= chunk) costs.push_back(2 * group * std::max(0, std::min(chunk, left)) + fixed);
+    }
+    pieces *= hkv;
+    slots *= hkv;
+    return static_cast<double>(pool_makespan(costs, hkv, per_cu)) + (slots ? pass + per_slot * static_cast<double>(slots) : 0.0);
+  };
+  int cap[2] = {kDkdvMaxBlocks, kDkdvMaxBlocks};
+  bool found = false;
+  // one cap for all tiles, then the suffix tiles' beside it, then the nodes'
+  for (int which : {2, 1, 0}) {
+    const int top = which == 2 ? std::max(longest[0], longest[1]) : longest[which];
+    const int at[2] = {cap[0], cap[1]};
+    int tried = 0;
+    for (int cut : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 64}) {
+      const int c = std::min<int>(kDkdvMaxBlocks, (top + cut - 1) / cut);
+      if (c == tried) continue;
+      tried = c;
+      const int node = which == 1 ? at[0] : c, suffix = which == 0 ? at[1] : c;
+      const double e = estimate(node, suffix);
+      if (slots <= 4 * units && e < best) {  // bounds the workspace: 134 MB, 101 MB at head_dim 64
+        best = e;
+        cap[0] = node;
+        cap[1] = suffix;
+        found = true;
+      }
+      if (slots > 4 * units || pieces > 8 * units) break;
+    }
+  }
+  if (!found) return out;
+  std::vector<Item> items;
+  for (const DkTile& t : tiles) {
+    const int n = dk_pieces(t, cap[t.src]), range = t.hi - t.lo, chunk = std::max(1, (range + n - 1) / n);
+    for (int h = 0; h < hkv; h++) {
+      if (chunk >= range) {
+        items.push_back({{t.src, t.seg, t.k0, h, t.lo, t.hi, -1, 0}, static_cast<int64_t>(range) * group + 1, h});
+        continue;
+      }
+      const int32_t slot0 = out.slots;
+      for (int32_t b = t.lo; b < t.hi; b += chunk) {
+        const int32_t e = std::min(t.hi, b + chunk);
+        items.push_back({{t.src, t.seg, t.k0, h, b, e, out.slots++, 0}, static_cast<int64_t>(e - b) * group + 1, h});
+      }
+      out.merges.insert(out.merges.end(), {t.src, t.seg, t.k0, h, slot0, out.slots - slot0, 0, 0});
+      out.n_merges++;
+    }
+  }
+  out.items = order_for_xcds(items, hkv, DK_WORDS, &out.n_items);
   return out;
 }
 
@@ -376,11 +457,9 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
         // keys the item streams: under a mask every suffix key may be visible
         const int64_t keys = prefix_len[s] + (masked ? len : std::min(tok + tokens, len));
         for (int qh = 0; qh < Hq; qh += heads) {
-          Item it;
-          it.words = {s, tok, qh, qh / G};
-          it.work = keys + (mfma_family ? static_cast<int64_t>(N - leaf_rank[s]) * (int64_t{1} << 40) : 0);
-          it.kvh = qh / G;
-          items.push_back(std::move(it));
+          items.push_back({{s, tok, qh, qh / G},
+                           keys + (mfma_family ? static_cast<int64_t>(N - leaf_rank[s]) * (int64_t{1} << 40) : 0),
+                           qh / G});
         }
       }
     }
@@ -425,31 +504,27 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
       }
     }
     if (chunk >= range || range == 0) {
-      Item it;
-      it.words = {src, seg, k0, h, lo, hi, -1, 0};
-      it.work = static_cast<int64_t>(range) * G + 1;
-      it.kvh = h;
-      dkdv.push_back(std::move(it));
+      dkdv.push_back({{src, seg, k0, h, lo, hi, -1, 0}, static_cast<int64_t>(range) * G + 1, h});
       return;
     }
     const int32_t slot0 = n_slots;
     int pieces = 0;
     for (int32_t b = lo; b < hi; b += chunk, pieces++) {
-      Item it;
-      it.words = {src, seg, k0, h, b, std::min(hi, b + chunk), n_slots++, 0};
-      it.work = static_cast<int64_t>(std::min(hi, b + chunk) - b) * G + 1;
-      it.kvh = h;
-      dkdv.push_back(std::move(it));
+      const int32_t e = std::min(hi, b + chunk);
+      dkdv.push_back({{src, seg, k0, h, b, e, n_slots++, 0}, static_cast<int64_t>(e - b) * G + 1, h});
     }
     red.insert(red.end(), {src, seg, k0, h, slot0, pieces, 0, 0});
     max_split = std::max(max_split, pieces);
   };
+  std::vector<DkTile> dk_tiles;
   for (int n = 0; n < M; n++) {
     const int len = no[n + 1] - no[n];
     // a node no leaf descends from gets an empty query range: its items write zeros
     const int32_t lo = leaf_qblk[leaf_lo[n]], hi = leaf_qblk[leaf_hi[n]];
-    for (int k0 = 0; k0 < len; k0 += KT)
+    for (int k0 = 0; k0 < len; k0 += KT) {
+      dk_tiles.push_back({0, n, k0, lo, hi});
       for (int h = 0; h < Hkv; h++) add_tile(0, n, k0, h, lo, hi);
+    }
   }
   // Suffix tiles: where one dK/dV workgroup fills a CU (the MFMA kernels at
   // head_dim 128 and 256), tile j of a leaf with T tiles is paired with its
@@ -467,16 +542,13 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
     for (int j = 0; j < tiles; j++) {
       const int mirror = tiles - 1 - j;
       const int lo_tile = std::min(j, mirror);   // the longer query range
+      dk_tiles.push_back({1, s, j * KT, first_block(j), leaf_qblk[s + 1]});
       if (pair_tiles && mirror != j && leaf_qblk[s + 1] - first_block(lo_tile) <= kDkdvMaxBlocks) {
         if (j == lo_tile) {
           const int32_t blocks = (leaf_qblk[s + 1] - first_block(j)) + (leaf_qblk[s + 1] - first_block(mirror));
-          for (int h = 0; h < Hkv; h++) {
-            Item it;
-            it.words = {1, s, mirror * KT, h, first_block(mirror), leaf_qblk[s + 1], -1, j * KT + 1};
-            it.work = static_cast<int64_t>(blocks) * G + 2;
-            it.kvh = h;
-            dkdv.push_back(std::move(it));
-          }
+          for (int h = 0; h < Hkv; h++)
+            dkdv.push_back({{1, s, mirror * KT, h, first_block(mirror), leaf_qblk[s + 1], -1, j * KT + 1},
+                            static_cast<int64_t>(blocks) * G + 2, h});
         }
         continue;
       }
@@ -487,6 +559,9 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   }
   int32_t n_dkdv = 0;
   std::vector<int32_t> dkdv_words = order_for_xcds(dkdv, Hkv, DK_WORDS, &n_dkdv);
+  Parts kparts;
+  if (mfma_family)
+    kparts = dkdv_parts(dk_tiles, dkdv, n_slots, Hkv, G, D == 64 ? 3 : 1, D == 256 ? 7 : 10, 5, D == 64 ? 0.02 : 0.09);
 
   // ---- dS store (bf16 head_dim 128 and 256) -------------------------------------
   // Every (key tile, query block) pair the dK/dV items stream gets one slot.
@@ -625,6 +700,7 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   };
   append_parts(fparts, PF_N_FPART, PF_OFF_FPART, PF_N_FMERGE, PF_OFF_FMERGE, PF_FSLOTS);
   append_parts(qparts, PF_N_QPART, PF_OFF_QPART, PF_N_QMERGE, PF_OFF_QMERGE, PF_QSLOTS);
+  append_parts(kparts, PF_N_KPART, PF_OFF_KPART, PF_N_KRED, PF_OFF_KRED, PF_KSLOTS);
   plan[PF_N_DQS] = n_dqs;
   plan[PF_OFF_DQS] = dqs_words.empty() ? 0 : append(dqs_words.data(), dqs_words.size());
   plan[PF_TOTAL_WORDS] = static_cast<int32_t>(plan.size());

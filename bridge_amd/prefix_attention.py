@@ -206,20 +206,29 @@ def _check_accumulators(accumulators, prefix_k) -> Tuple[torch.Tensor, torch.Ten
 
 
 def _workspace(meta, q, k, budget, ws, masked=False):
-    """(plan, workspace) of the backward. A plan with a dS store whose
-    workspace cannot be allocated falls back to the plan without one (a few
-    MB), which gives the same gradients with a slower dQ."""
+    """(plan, workspace, its bytes) of the backward. A given workspace is the
+    plan's ``workspace_bytes``; one allocated here has room for the dK/dV parts
+    too. Where that cannot be allocated the backward runs without the parts,
+    and a plan with a dS store falls back to the plan without one (a few MB),
+    which gives the same gradients with a slower dQ."""
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=budget, masked=masked)
-    if ws is not None or not plan.workspace_bytes:
-        return plan, ws
+    if ws is not None:
+        return plan, ws, plan.workspace_bytes
+    if plan.bwd_parts_bytes > plan.workspace_bytes:
+        try:
+            return plan, torch.empty(plan.bwd_parts_bytes, dtype=torch.uint8, device=q.device), plan.bwd_parts_bytes
+        except torch.OutOfMemoryError:
+            pass
+    if not plan.workspace_bytes:
+        return plan, None, 0
     try:
-        return plan, torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=q.device)
+        return plan, torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=q.device), plan.workspace_bytes
     except torch.OutOfMemoryError:
         if not plan.dq_from_ds:
             raise
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
     ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=q.device) if plan.workspace_bytes else None
-    return plan, ws
+    return plan, ws, plan.workspace_bytes
 
 
 def _backward(q, k, v, prefix_k, prefix_v, out, lse, dout, meta, scale, *, phases=None, buffers=None,
@@ -251,13 +260,13 @@ def _backward(q, k, v, prefix_k, prefix_v, out, lse, dout, meta, scale, *, phase
             return dq, dk, dv, dpk, dpv
         return dq, dk, dv, dpk.zero_(), dpv.zero_()
     delta = b.get("delta") if b.get("delta") is not None else torch.empty_like(lse)
-    plan, ws = _workspace(meta, q, k, ds_store_budget, b.get("workspace"), masked=mask is not None)
+    plan, ws, ws_bytes = _workspace(meta, q, k, ds_store_budget, b.get("workspace"), masked=mask is not None)
     lib = _lib.load()
     params = _lib.TprBwdParams(
         _lib.ABI_VERSION, flags, scale, 0.0,
         plan.host.data_ptr(), plan.device.data_ptr(),
         _ptr(q), _ptr(k), _ptr(v), _ptr(prefix_k), _ptr(prefix_v), _ptr(out), _ptr(dout), _ptr(lse),
-        _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dpk), _ptr(dpv), _ptr(ws), plan.workspace_bytes,
+        _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dpk), _ptr(dpv), _ptr(ws), ws_bytes,
         _row_stride(q), _row_stride(k), _row_stride(v), *_mask_args(mask))
     mask = phases if phases is not None else (_lib.TPR_BWD_DELTA | _lib.TPR_BWD_DKDV | _lib.TPR_BWD_DQ)
     _lib.check(lib.tpr_attn_bwd_phases(ctypes.byref(params), int(mask), ctypes.c_void_p(_stream_handle(q.device))),
