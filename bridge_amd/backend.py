@@ -163,9 +163,10 @@ class TPRKernelBackend:
         accumulators = None
         if self._accumulators is not None and self._prefix_length:
             accumulators = self._accumulators[layer_number]
-        out, _ = TPRPrefixAttention.apply(query[:, 0], new_key[:, 0], new_value[:, 0], past_key[:, 0],
-                                          past_value[:, 0], self._meta, softmax_scale, accumulators, False,
-                                          self._ds_store_budget)
+        # squeeze: the backward of an index would fill and copy each gradient
+        out, _ = TPRPrefixAttention.apply(query.squeeze(1), new_key.squeeze(1), new_value.squeeze(1),
+                                          past_key.squeeze(1), past_value.squeeze(1), self._meta, softmax_scale,
+                                          accumulators, False, self._ds_store_budget)
         return out.reshape(query.shape[0], 1, query.shape[2] * query.shape[3])
 
     # -- packing helpers --------------------------------------------------------

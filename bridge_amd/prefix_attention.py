@@ -315,6 +315,7 @@ class TPRPrefixAttention(torch.autograd.Function):
         ctx.accumulators = prefix_grad_accumulators
         ctx.ds_store_budget = budget
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)  # no zeros for lse
         return out, lse
 
     @staticmethod

@@ -30,7 +30,7 @@ import torch
 from torch import Tensor
 
 from .meta import TPRPrefixMeta
-from .prefix_attention import TPRPrefixAttention
+from .prefix_attention import _backward, _forward, _inputs, check_mask, validate
 
 __all__ = ["rectangular_causal_attention"]
 
@@ -94,6 +94,34 @@ def _single_leaf_meta(prefix_length: int, query_length: int) -> TPRPrefixMeta:
     return TPRPrefixMeta.shared_prefix(prefix_length, [query_length])
 
 
+class _RectangularAttention(torch.autograd.Function):
+    """``TPRPrefixAttention`` of one leaf whose prefix and suffix are the rows of
+    one K and one V tensor: the kernels write both parts' gradients into one
+    buffer. (With the rows sliced outside, autograd filled, copied and added
+    each part's gradient: 55 us at 3072 x 8 x 128.)"""
+
+    @staticmethod
+    def forward(ctx, q, k, v, meta, scale, attention_mask):
+        p = meta.total_prefix
+        rows = (q, k[p:], v[p:], k[:p], v[:p])
+        scale = validate(*rows, meta, scale)
+        mask = check_mask(attention_mask, q, meta)
+        rows = _inputs(*rows)
+        out, lse = _forward(*rows, meta, scale, mask)
+        ctx.save_for_backward(*rows, out, lse)
+        ctx.mask, ctx.meta, ctx.scale = mask, meta, scale
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        q, k, v, prefix_k, prefix_v, out, lse = ctx.saved_tensors
+        p = ctx.meta.total_prefix
+        dk, dv = (torch.empty((p + k.shape[0], *k.shape[1:]), dtype=k.dtype, device=k.device) for _ in range(2))
+        dq = _backward(q, k, v, prefix_k, prefix_v, out, lse, dout.contiguous(), ctx.meta, ctx.scale, mask=ctx.mask,
+                       buffers={"dk": dk[p:], "dv": dv[p:], "dprefix_k": dk[:p], "dprefix_v": dv[:p]})[0]
+        return dq, dk, dv, None, None, None
+
+
 def rectangular_causal_attention(
     query: Tensor,
     key: Tensor,
@@ -135,9 +163,7 @@ def rectangular_causal_attention(
     v = value.squeeze(1)
     meta = _single_leaf_meta(prefix_length, query_length)
     # one leaf: the mask's columns cat(prefix, suffix) are the leaf's key sequence
-    output, _ = TPRPrefixAttention.apply(q[:, :, :], k[prefix_length:], v[prefix_length:],
-                                         k[:prefix_length], v[:prefix_length], meta, softmax_scale,
-                                         None, False, None, attention_mask)
+    output = _RectangularAttention.apply(q, k, v, meta, softmax_scale, attention_mask)
     expected_shape = (query_length, query_heads, head_dim)
     if tuple(output.shape) != expected_shape:
         raise RuntimeError(f"unexpected attention output shape: expected {expected_shape}, got {tuple(output.shape)}")
