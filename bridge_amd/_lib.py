@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "tpr_attn_bwd_phases",
     "tpr_attn_bwd_noalloc",
     "tpr_attn_bwd_noalloc_max_workspace_bytes",
+    "tpr_attn_mask_differs_from_causal",
 )
 
 TPR_BWD_DELTA = 1
@@ -171,6 +172,8 @@ def load():
         lib.tpr_attn_bwd_noalloc.argtypes = [ctypes.POINTER(TprBwdParams), _p]
         lib.tpr_attn_bwd_noalloc_max_workspace_bytes.restype = ctypes.c_size_t
         lib.tpr_attn_bwd_noalloc_max_workspace_bytes.argtypes = []
+        lib.tpr_attn_mask_differs_from_causal.restype = ctypes.c_int
+        lib.tpr_attn_mask_differs_from_causal.argtypes = [_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _p, _p]
         version = lib.tpr_attn_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}; rebuild it")

@@ -495,3 +495,46 @@ extern "C" int tpr_attn_bwd_noalloc(const TprBwdParams* p, void* stream) {
   const size_t bytes = std::min(kScratchBytes, tpr_attn_bwd_workspace_bytes(p->plan_host));
   return bwd_phases(p, TPR_BWD_DELTA | TPR_BWD_DKDV | TPR_BWD_DQ, stream, ws, bytes);
 }
+
+// ---------------------------------------------------------------------------
+// Whether a [rows, cols] byte mask (nonzero = hidden) is not the right-down
+// causal one. One workgroup per row, 16 bytes a lane at any alignment; bound by
+// the one read of the mask. Lanes that see a difference store the same 1.
+namespace tpr {
+namespace {
+__global__ __launch_bounds__(256) void mask_differs(const uint8_t* mask, int64_t row_stride, int rows, int cols,
+                                                    int32_t* flag) {
+  const uint8_t* m = mask + static_cast<int64_t>(blockIdx.x) * row_stride;
+  const int visible = cols - rows + static_cast<int>(blockIdx.x) + 1;  // leading columns the row sees
+  uint32_t diff = 0;
+  for (int64_t c = 16 * static_cast<int>(threadIdx.x); c < cols; c += 16 * 256) {
+    if (c + 16 <= cols) {
+      uint32_t w[4];
+      __builtin_memcpy(w, m + c, 16);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t hidden = (((w[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[i]) & 0x80808080u;
+        const int64_t seen = visible - (c + 4 * i);
+        diff |= hidden ^ (seen >= 4 ? 0u : seen <= 0 ? 0x80808080u : 0x80808080u << (8 * seen));
+      }
+    } else {
+      for (int64_t j = c; j < cols; j++) diff |= (m[j] != 0) != (j >= visible) ? 1u : 0u;
+    }
+  }
+  if (diff) *flag = 1;
+}
+}  // namespace
+}  // namespace tpr
+
+extern "C" int tpr_attn_mask_differs_from_causal(const uint8_t* mask, int64_t row_stride, int32_t rows, int32_t cols,
+                                            int32_t* flag, void* stream) {
+  clear_error();
+  if (!mask || !flag) return fail(TPR_ERR_INVALID_ARGUMENT, "mask and flag must not be NULL");
+  if (rows <= 0 || cols < rows || row_stride < (rows > 1 ? cols : 0))
+    return fail(TPR_ERR_INVALID_ARGUMENT, "a mask needs 0 < rows <= cols <= row stride, got %d, %d, %lld", rows, cols,
+                static_cast<long long>(row_stride));
+  hipLaunchKernelGGL(mask_differs, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream), mask, row_stride, rows, cols,
+                     flag);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? TPR_OK : fail(TPR_ERR_LAUNCH, "mask check launch failed: %s", hipGetErrorString(e));
+}

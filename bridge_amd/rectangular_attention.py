@@ -23,12 +23,14 @@ kernels. A query row the mask hides entirely gets output 0 and no gradient.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from functools import lru_cache
 
 import torch
 from torch import Tensor
 
+from . import _lib
 from .meta import TPRPrefixMeta
 from .prefix_attention import _backward, _forward, _inputs, check_mask, validate
 
@@ -82,11 +84,17 @@ def _validate_attention_mask(attention_mask, *, query_length: int, kv_length: in
         raise ValueError(f"attention_mask must have shape {expected}, got {tuple(attention_mask.shape)}")
 
 
-def _right_down_causal_mask(query_length: int, kv_length: int, device) -> Tensor:
-    """True = excluded: key j is hidden from query i iff j > kv_length - query_length + i."""
-    cols = torch.arange(kv_length, device=device)
-    rows = torch.arange(query_length, device=device)
-    return cols[None, :] > (kv_length - query_length + rows[:, None])
+def _is_right_down_causal(mask: Tensor) -> bool:
+    """Whether a GPU mask is the right-down causal one (key j hidden from query
+    i iff j > Skv - Sq + i), read once by a kernel. (Built and compared with
+    torch.equal it took 45 us of kernels at 2048 x 3072, then the same wait.)"""
+    if mask.stride(1) != 1 or mask.stride(0) < mask.shape[1]:
+        mask = mask.contiguous()
+    flag = torch.zeros(1, dtype=torch.int32, device=mask.device)
+    _lib.check(_lib.load().tpr_attn_mask_differs_from_causal(
+        mask.data_ptr(), mask.stride(0), mask.shape[0], mask.shape[1], flag.data_ptr(),
+        ctypes.c_void_p(torch.cuda.current_stream(mask.device).cuda_stream)), "tpr_attn_mask_differs_from_causal")
+    return int(flag.item()) == 0
 
 
 @lru_cache(maxsize=256)
@@ -153,8 +161,7 @@ def rectangular_causal_attention(
         raise ValueError(f"softmax_scale must be finite and positive, got {softmax_scale}")
     if pre_tokens < kv_length:
         raise NotImplementedError("a preceding-token window shorter than the KV length is not supported")
-    if attention_mask is not None and torch.equal(
-            attention_mask, _right_down_causal_mask(query_length, kv_length, attention_mask.device)):
+    if attention_mask is not None and _is_right_down_causal(attention_mask):
         attention_mask = None  # the causal mask itself: the unmasked kernels
 
     prefix_length = kv_length - query_length

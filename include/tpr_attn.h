@@ -285,6 +285,13 @@ int tpr_attn_bwd_noalloc(const TprBwdParams* params, void* stream);
 /* Bytes of static scratch tpr_attn_bwd_noalloc has per GPU. */
 size_t tpr_attn_bwd_noalloc_max_workspace_bytes(void);
 
+/* Sets *flag (device memory, zeroed by the caller) to 1 if a [rows, cols] byte
+ * mask (device memory, nonzero = hidden, rows row_stride bytes apart, rows <=
+ * cols) is not the right-down causal one: column j hidden from row i iff
+ * j > cols - rows + i. Enqueued on `stream`. */
+int tpr_attn_mask_differs_from_causal(const uint8_t* mask, int64_t row_stride, int32_t rows, int32_t cols,
+                                 int32_t* flag, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,6 +1,7 @@
 """GPU: rectangular_causal_attention against the packed operator it stands on,
 called on row slices of the same tensors: outputs and gradients are the same
-bit for bit, for packed and strided K/V, with and without a prefix or a mask."""
+bit for bit, for packed and strided K/V, with and without a prefix or a mask;
+and the check that sends the right-down causal mask to the unmasked kernels."""
 
 from __future__ import annotations
 
@@ -40,3 +41,23 @@ def test_rect_equals_sliced_prefix_attention(sq, skv, d, dtype, masked, strided,
     assert torch.equal(out, ref.reshape(out.shape))
     for name, a, b in zip(("dq", "dk", "dv"), grads, want):
         assert a.shape == b.shape and torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("sq, skv", [(1, 1), (1, 50), (37, 37), (64, 128), (33, 4099), (300, 517)])
+def test_causal_mask_check_sees_every_element(sq, skv, cuda_device):
+    from bridge_amd.rectangular_attention import _is_right_down_causal
+    cols, rows = torch.arange(skv), torch.arange(sq)
+    mask = cols[None, :] > (skv - sq + rows[:, None])
+    at = mask.to(cuda_device)
+    assert _is_right_down_causal(at)
+    assert _is_right_down_causal(mask.t().contiguous().to(cuda_device).t())                 # columns strided
+    wide = torch.ones(sq, skv + 5, dtype=torch.bool, device=cuda_device)
+    wide[:, 3:skv + 3] = at
+    assert _is_right_down_causal(wide[:, 3:skv + 3])                                         # rows strided, odd start
+    gen = torch.Generator().manual_seed(sq * skv)
+    spots = {(0, 0), (sq - 1, skv - 1), (0, skv - 1), (sq - 1, 0)}
+    spots |= {(int(torch.randint(sq, (1,), generator=gen)), int(torch.randint(skv, (1,), generator=gen))) for _ in range(20)}
+    for r, c in sorted(spots):
+        other = at.clone()
+        other[r, c] = ~other[r, c]
+        assert not _is_right_down_causal(other), (r, c)
