@@ -33,7 +33,7 @@ EXPORTED_SYMBOLS = (
     "tpr_attn_last_error",
     "tpr_attn_plan",
     "tpr_attn_bwd_workspace_bytes",
-    "tpr_attn_bwd_parts_workspace_bytes",
+    "tpr_attn_bwd_min_workspace_bytes",
     "tpr_attn_fwd",
     "tpr_attn_fwd_ws",
     "tpr_attn_fwd_workspace_bytes",
@@ -156,8 +156,8 @@ def load():
                                       ctypes.POINTER(ctypes.c_int64)]
         lib.tpr_attn_bwd_workspace_bytes.restype = ctypes.c_size_t
         lib.tpr_attn_bwd_workspace_bytes.argtypes = [_p]
-        lib.tpr_attn_bwd_parts_workspace_bytes.restype = ctypes.c_size_t
-        lib.tpr_attn_bwd_parts_workspace_bytes.argtypes = [_p]
+        lib.tpr_attn_bwd_min_workspace_bytes.restype = ctypes.c_size_t
+        lib.tpr_attn_bwd_min_workspace_bytes.argtypes = [_p]
         lib.tpr_attn_fwd.restype = ctypes.c_int
         lib.tpr_attn_fwd.argtypes = [ctypes.POINTER(TprFwdParams), _p]
         lib.tpr_attn_fwd_ws.restype = ctypes.c_int

@@ -1,7 +1,6 @@
 // tpr_abi.hip -- extern "C" entry points of libtpr_attn.so: argument checks,
 // plan-header decoding and kernel dispatch. Host code only.
 
-#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -255,12 +254,12 @@ size_t fpart_bytes(const int32_t* ph) {
 
 extern "C" size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host) {
   if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
-  return bwd_base_bytes(plan_host) + qpart_bytes(plan_host);
+  return bwd_base_bytes(plan_host) + qpart_bytes(plan_host) + kpart_bytes(plan_host);
 }
 
-extern "C" size_t tpr_attn_bwd_parts_workspace_bytes(const int32_t* plan_host) {
+extern "C" size_t tpr_attn_bwd_min_workspace_bytes(const int32_t* plan_host) {
   if (!plan_host || plan_host[PF_MAGIC] != kPlanMagic) return 0;
-  return bwd_base_bytes(plan_host) + qpart_bytes(plan_host) + kpart_bytes(plan_host);
+  return bwd_base_bytes(plan_host);
 }
 
 extern "C" size_t tpr_attn_fwd_workspace_bytes(const int32_t* plan_host) {
@@ -490,10 +489,7 @@ extern "C" int tpr_attn_bwd_noalloc(const TprBwdParams* p, void* stream) {
   void* ws = nullptr;
   int rc = scratch_for_current_device(static_cast<hipStream_t>(stream), &ws);
   if (rc) return rc;
-  // as tpr_attn_bwd with that many bytes runs: whole dK/dV items, and dQ's key
-  // parts where the scratch holds them
-  const size_t bytes = std::min(kScratchBytes, tpr_attn_bwd_workspace_bytes(p->plan_host));
-  return bwd_phases(p, TPR_BWD_DELTA | TPR_BWD_DKDV | TPR_BWD_DQ, stream, ws, bytes);
+  return bwd_phases(p, TPR_BWD_DELTA | TPR_BWD_DKDV | TPR_BWD_DQ, stream, ws, kScratchBytes);
 }
 
 // ---------------------------------------------------------------------------

@@ -198,7 +198,8 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
 // run (prefix 738 + 3016 + 905, GQA 16/2: 54 items, 14 % of the chip busy). The
 // query ranges are then cut into parts of at most `cap` blocks, one cap for
 // node tiles and one for suffix tiles (which then run unpaired), whose fp32
-// partial tiles the reduction pass sums in query-block order.
+// partial tiles the reduction pass sums in query-block order. Only where the
+// whole items leave no partials: a workspace holds one set of slots.
 struct DkTile {
   int32_t src, seg, k0, lo, hi;
 };
@@ -207,7 +208,7 @@ int dk_pieces(const DkTile& t, int cap) { return std::max(1, (t.hi - t.lo + cap 
 // Costs in half head-blocks (64 queries of one head against one key tile; 1.0
 // us at head_dim 128, 1.4 at 256, 0.9 at 64): `fixed` a workgroup's start and
 // end, `pass` the reduction launch, `per_slot` writing and reading a partial.
-Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base, int32_t base_slots, int hkv, int group,
+Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base, int hkv, int group,
                  int per_cu, int fixed, double pass, double per_slot) {
   Parts out;
   const int units = kPlanCus * per_cu;
@@ -220,7 +221,7 @@ Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base
       total += costs.back();
     }
   if (costs.empty()) return out;
-  double best = 0.92 * (static_cast<double>(pool_makespan(costs, hkv, per_cu)) + (base_slots ? pass + per_slot * base_slots : 0.0));
+  double best = 0.92 * static_cast<double>(pool_makespan(costs, hkv, per_cu));
   // a launch this well balanced already is not worth more partials
   if (static_cast<double>(total) * hkv / units >= best) return out;
   int longest[2] = {1, 1};
@@ -560,8 +561,8 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
   int32_t n_dkdv = 0;
   std::vector<int32_t> dkdv_words = order_for_xcds(dkdv, Hkv, DK_WORDS, &n_dkdv);
   Parts kparts;
-  if (mfma_family)
-    kparts = dkdv_parts(dk_tiles, dkdv, n_slots, Hkv, G, D == 64 ? 3 : 1, D == 256 ? 7 : 10, 5, D == 64 ? 0.02 : 0.09);
+  if (mfma_family && n_slots == 0)
+    kparts = dkdv_parts(dk_tiles, dkdv, Hkv, G, D == 64 ? 3 : 1, D == 256 ? 7 : 10, 5, D == 64 ? 0.02 : 0.09);
 
   // ---- dS store (bf16 head_dim 128 and 256) -------------------------------------
   // Every (key tile, query block) pair the dK/dV items stream gets one slot.

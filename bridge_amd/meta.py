@@ -59,7 +59,7 @@ class LaunchPlan:
     device: torch.Tensor   # int32, on the compute device
     workspace_bytes: int          # backward
     fwd_workspace_bytes: int = 0  # forward key parts (few query rows), else 0
-    bwd_parts_bytes: int = 0      # the backward's with room for its dK/dV parts (>= workspace_bytes)
+    bwd_min_bytes: Optional[int] = None  # the backward's without its parts (None: workspace_bytes)
 
     @property
     def path(self) -> str:
@@ -287,6 +287,6 @@ class TPRPrefixMeta:
         at = ctypes.c_void_p(host.data_ptr())
         plan = LaunchPlan(host, dev, int(lib.tpr_attn_bwd_workspace_bytes(at)),
                           int(lib.tpr_attn_fwd_workspace_bytes(at)),
-                          int(lib.tpr_attn_bwd_parts_workspace_bytes(at)))
+                          int(lib.tpr_attn_bwd_min_workspace_bytes(at)))
         self._plans[key] = plan
         return plan

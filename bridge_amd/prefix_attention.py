@@ -206,29 +206,28 @@ def _check_accumulators(accumulators, prefix_k) -> Tuple[torch.Tensor, torch.Ten
 
 
 def _workspace(meta, q, k, budget, ws, masked=False):
-    """(plan, workspace, its bytes) of the backward. A given workspace is the
-    plan's ``workspace_bytes``; one allocated here has room for the dK/dV parts
-    too. Where that cannot be allocated the backward runs without the parts,
-    and a plan with a dS store falls back to the plan without one (a few MB),
-    which gives the same gradients with a slower dQ."""
+    """(plan, workspace, its bytes) of the backward. Where the workspace cannot
+    be allocated the backward runs without its parts, and a plan with a dS
+    store falls back to the plan without one (a few MB), which gives the same
+    gradients with a slower dQ."""
+    def empty(size):
+        return torch.empty(size, dtype=torch.uint8, device=q.device) if size else None
+
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=budget, masked=masked)
     if ws is not None:
         return plan, ws, plan.workspace_bytes
-    if plan.bwd_parts_bytes > plan.workspace_bytes:
-        try:
-            return plan, torch.empty(plan.bwd_parts_bytes, dtype=torch.uint8, device=q.device), plan.bwd_parts_bytes
-        except torch.OutOfMemoryError:
-            pass
-    if not plan.workspace_bytes:
-        return plan, None, 0
-    try:
-        return plan, torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=q.device), plan.workspace_bytes
-    except torch.OutOfMemoryError:
-        if not plan.dq_from_ds:
-            raise
-    plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
-    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=q.device) if plan.workspace_bytes else None
-    return plan, ws, plan.workspace_bytes
+    plans = [plan]
+    if plan.dq_from_ds:
+        plans.append(None)  # the plan without a store, built only if needed
+    for p in plans:
+        p = p or meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
+        least = p.workspace_bytes if p.bwd_min_bytes is None else p.bwd_min_bytes
+        for size in sorted({p.workspace_bytes, least}, reverse=True):
+            try:
+                return p, empty(size), size
+            except torch.OutOfMemoryError as exc:
+                error = exc
+    raise error
 
 
 def _backward(q, k, v, prefix_k, prefix_v, out, lse, dout, meta, scale, *, phases=None, buffers=None,

@@ -224,13 +224,13 @@ int tpr_attn_plan(const TprTreeDesc* tree, int32_t* plan, int64_t capacity_words
  * partial sums, and the dS store of a plan that has one). */
 size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host);
 
-/* The same with room for the dK/dV parts: with at least this much workspace, a
- * tree whose key tiles are too few or too uneven to fill the GPU has their
- * query ranges cut over more workgroups (summed in query order; dK/dV may
- * round differently in the last bits). Equal to tpr_attn_bwd_workspace_bytes()
- * for a plan without parts. The phases of one backward must all be given the
- * same workspace_bytes. */
-size_t tpr_attn_bwd_parts_workspace_bytes(const int32_t* plan_host);
+/* The least the backward runs with. Where rows or key tiles are too few or too
+ * uneven to fill the GPU, a plan also cuts dQ along the keys and dK/dV along
+ * the queries over more workgroups; with less than
+ * tpr_attn_bwd_workspace_bytes() those parts do not run (the sums' order, and
+ * so the last bits, differ). All phases of one backward must be given the same
+ * workspace_bytes. */
+size_t tpr_attn_bwd_min_workspace_bytes(const int32_t* plan_host);
 
 /* Enqueue the forward on `stream` (a hipStream_t; NULL = default stream). */
 int tpr_attn_fwd(const TprFwdParams* params, void* stream);

@@ -11,7 +11,9 @@ delta from the rounded output, and dP - delta cancels where a row has few keys
 
 from __future__ import annotations
 
+import dataclasses
 import math
+from unittest import mock
 
 import pytest
 import torch
@@ -46,20 +48,21 @@ def test_dkdv_parts_match_oracle_and_whole_items(name, d, recompute, relay, cuda
     hq, hkv = (6, 2) if name == "ragged" else (4, 2)
     scale = 1.0 / math.sqrt(d)
     plan = meta.plan(hq, hkv, d, torch.bfloat16, cuda_device, recompute_dq=recompute)
-    assert plan.host[N_KPART] > 0 and plan.bwd_parts_bytes > plan.workspace_bytes
+    assert plan.host[N_KPART] > 0 and plan.workspace_bytes > plan.bwd_min_bytes
     q, k, v, pk, pv, dout = make_inputs(meta, hq, hkv, d, torch.bfloat16, seed=11 + d, device=cuda_device)
     print(f"[dK/dV parts {name} d{d} recompute={recompute} relay={relay}] {int(plan.host[N_KPART])} items, "
           f"{int(plan.host[N_KPART + 4])} slots", flush=True)
     out, lse = prefix_attention_forward(q, k, v, pk, pv, meta, scale)
 
-    def backward(**more):
+    def backward(sized):
         acc = tuple(torch.full(pk.shape, 0.25, dtype=torch.float32, device=cuda_device) for _ in range(2)) if relay else None
-        return prefix_attention_backward(q, k, v, pk, pv, out, lse, dout, meta, scale, recompute_dq=recompute,
-                                         prefix_grad_accumulators=acc, **more)
+        ws = torch.empty(sized.workspace_bytes, dtype=torch.uint8, device=cuda_device)
+        with mock.patch.object(type(meta), "plan", return_value=sized):
+            return prefix_attention_backward(q, k, v, pk, pv, out, lse, dout, meta, scale, recompute_dq=recompute,
+                                             prefix_grad_accumulators=acc, buffers={"workspace": ws})
 
-    parts, again = backward(), backward()
-    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=cuda_device)
-    whole = backward(buffers={"workspace": ws})
+    parts, again = backward(plan), backward(plan)
+    whole = backward(dataclasses.replace(plan, workspace_bytes=plan.bwd_min_bytes))
     torch.cuda.synchronize()
     _, _, ref = oracle(meta, q, k, v, pk, pv, dout, scale)
     for i, label in enumerate(("dq", "dk", "dv", "dprefix_k", "dprefix_v")):
