@@ -169,7 +169,7 @@ constexpr int kDsHeadBytes = kDkdvKeys * kDkdvQ * 2;          // 16 KiB per quer
 // (query head, token) in the lse layout, then -delta in the same layout.
 constexpr int kStatRowsOffset = 64;   // floats before the lse*log2e rows
 // MFMA16 family (bf16, head_dim 64 and 256)
-constexpr int kM16Waves = 4;          // waves per workgroup (all kernels)
+constexpr int kM16Waves = 4;          // waves per workgroup (8 in some kernels at head_dim 256)
 constexpr int kM16Tokens = 32;        // forward / dQ tokens per wave (two 16-query sub-blocks)
 constexpr int kM16DqsWaves = 8;       // waves of the head_dim-256 dQ-from-store workgroup (two per SIMD)
 // dK/dV keys per wave: one 16-key block (at head_dim 256 the accumulators of

@@ -103,6 +103,9 @@ __device__ __forceinline__ bf16x8 col_operand(const char* tile, int r0, int c0, 
   return r;
 }
 
+// waves of a dK/dV workgroup (two per SIMD at head_dim 256)
+constexpr int m16_dkdv_waves(int d) { return d == 256 ? 2 * kM16Waves : kM16Waves; }
+
 // Copy rows [0, 64) of the tile whose row 0 is at `src` (uniform; rows at or
 // beyond `len` re-read row len - 1; row stride `stride` bytes) into the
 // swizzled LDS tile at `lds_tile`: this wave's BPW 1 KiB blocks. Lane l of
@@ -1014,8 +1017,9 @@ __global__ __launch_bounds__(kD) void m16_dq_merge(KernelArgs a, int hpw, int sl
 }
 
 // ---------------------------------------------------------------------------
-// dK/dV. One workgroup = 4 waves x 16 keys (KB 16-key blocks kb per wave) of
-// one KV segment tile and KV head; it streams every 64-query block that
+// dK/dV. One workgroup = 4 waves x 16 keys (KB 16-key blocks kb per wave; 8
+// waves at head_dim 256, two for each 16 keys) of one KV segment tile and KV
+// head; it streams every 64-query block that
 // sees the tile -- for a prefix node every descendant leaf and every query
 // head of the group -- in the plan's fixed order, so a prefix node's gradient
 // is the sum over its leaves in registers, without atomics. Per stage (one
@@ -1029,10 +1033,22 @@ __global__ __launch_bounds__(kD) void m16_dq_merge(KernelArgs a, int hpw, int sl
 // kStrided as in m16_fwd; kStoreDs: also store every dS block to the dS store
 // (a.ds, head_dim 256) for the dQ kernel
 template <int kD, bool kStrided, bool kStoreDs>
-__global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
+__global__ __launch_bounds__(64 * m16_dkdv_waves(kD)) void m16_dkdv(KernelArgs a) {
   using T = Geo<kD>;
   constexpr int kWaveKeys = m16_wave_keys(kD);
   constexpr int kKeys = m16_keys(kD);
+  // head_dim 256: two waves share 16 keys, two waves a SIMD. Each takes 32 of a
+  // block's 64 queries in the S / dP products and 128 of the 256 columns of dK
+  // and dV, and they hand each other P and dS through LDS. One wave for 16 keys
+  // (one a SIMD) waited on its own LDS reads, 128 KB a stage at 35 to 51 bytes a
+  // cycle beside 2048 cycles of MFMA; now the unit's 512 KB of LDS reads a stage
+  // bound it. A layer pass at prefix 4096 + 4 x 4096, GQA 8/2: 3386 -> 3300 us.
+  // (Four waves, two sharing 32 keys: half the LDS reads, but one wave a SIMD
+  // again, 3584 us.)
+  constexpr bool kShare = kD == 256;
+  constexpr int kW = m16_dkdv_waves(kD);
+  static_assert(!kShare || kWaveKeys == 16, "one 16-key block per pair of waves");
+  constexpr int ND = kShare ? T::ND / 2 : T::ND;  // 16-column blocks of dK / dV per wave
   constexpr int KB = kWaveKeys / 16;  // 16-key blocks per wave
   const int32_t* item = a.plan + a.off_dkdv + DK_WORDS * blockIdx.x;
   if (item[DK_SRC] < 0) return;
@@ -1046,6 +1062,7 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i16 = lane & 15, g = lane >> 4;
+  const int kgroup = kShare ? wave >> 1 : wave, half = kShare ? wave & 1 : 0;
 
   const int64_t kstride = static_cast<int64_t>(a.hkv) * kD;  // packed K/V rows: prefix inputs, every output
   const uint32_t g_rb = static_cast<uint32_t>(a.hq) * kD * 2;  // dO row bytes (packed)
@@ -1054,6 +1071,8 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[2 * 2 * T::TB];           // [buf][Q | dO]
   __shared__ __attribute__((aligned(256))) float stats[2][2][kTileRows];       // [buf][-lse*log2e | -delta][row]
   __shared__ int4 qtab[kDkdvMaxBlocks];
+  // P and dS handed over: [key group][query half][P | dS][lane]
+  __shared__ __attribute__((aligned(1024))) bf16x8 hand[kShare ? 4 * 2 * 2 * 64 : 1];
 
   // An item is one key tile, or two suffix tiles of one leaf (DK_PAIR), a
   // tile and its mirror: the first streams its query blocks last-first, the
@@ -1067,7 +1086,7 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
     const int qb_hi = item[DK_QB_HI];
     const int qb_lo = tile == 0 ? item[DK_QB_LO] : item[DK_QB_LO] - (item[DK_KEY0] - key0) / kTileRows;
     const bool first_last = prefix || tile == 1;
-    const int kw0 = key0 + kWaveKeys * wave;  // first key position of this wave
+    const int kw0 = key0 + kWaveKeys * kgroup;  // first key position of this wave
     const bool wave_active = kw0 < seg_len;
 
     if (tile > 0) __syncthreads();  // every wave is done with the previous tile's table
@@ -1095,8 +1114,8 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
       const int64_t goff = col + static_cast<int64_t>(row) * g_rb;
       const int64_t qoff = kStrided ? col + static_cast<int64_t>(row) * q_rb : goff;
       const uint32_t tile = lds0 + buf * 2 * T::TB;
-      copy_tile<kD>(reinterpret_cast<const char*>(a.q) + qoff, q_rb, nq, tile, wave, lane);
-      copy_tile<kD>(reinterpret_cast<const char*>(a.dout) + goff, g_rb, nq, tile + T::TB, wave, lane);
+      copy_tile<kD, kW>(reinterpret_cast<const char*>(a.q) + qoff, q_rb, nq, tile, wave, lane);
+      copy_tile<kD, kW>(reinterpret_cast<const char*>(a.dout) + goff, g_rb, nq, tile + T::TB, wave, lane);
       if (wave < 2) {  // wave 0: -lse*log2e, wave 1: -delta; rows past the block end copy -inf / 0
         const int64_t at = static_cast<int64_t>(qh) * a.total_q + row + lane;
         const float* rows = wave == 0 ? a.stat_ws + kStatRowsOffset : a.ndelta_ws;
@@ -1123,11 +1142,11 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
       }
     }
     // register r of block [kb][db]: key 16 kb + 4 g + r of the wave, head dim 16 db + l % 16
-    f32x4 dk[KB][T::ND], dv[KB][T::ND];
+    f32x4 dk[KB][ND], dv[KB][ND];
 #pragma unroll
     for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-      for (int db = 0; db < T::ND; db++) {
+      for (int db = 0; db < ND; db++) {
         dk[kb][db] = f32x4{};
         dv[kb][db] = f32x4{};
       }
@@ -1154,7 +1173,7 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
           const int slot = __builtin_amdgcn_readfirstlane(qtab[blk].w);
           ds_stage = static_cast<char*>(a.ds) +
                      ((static_cast<int64_t>(kvh) * a.ds_slots + slot) * group + sidx % group) * m16_ds_head_bytes(kD) +
-                     wave * (m16_ds_head_bytes(kD) / kM16Waves);
+                     kgroup * (m16_ds_head_bytes(kD) / kM16Waves);
         }
         const char* qt = smem + buf * 2 * T::TB;
         const char* gt = qt + T::TB;
@@ -1162,6 +1181,87 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
         const float* ndel = &stats[buf][1][0];
         // query q of the block visible from key kp iff kp <= tok0 + q (suffix tiles)
         const bool diag = !prefix && tok0 < kw0 + kWaveKeys - 1;
+        bf16x8 pT[KB], dT[KB];  // queries 32 t + 8 g + 0..7 of key 16 kb + l % 16
+        if constexpr (kShare) {
+          // S and dP of the 16 keys and the wave's half of the queries, one fenced
+          // slot per 32 dims; operands are read kAhead1 slots ahead
+          constexpr int kAhead1 = 2, kRing1 = kAhead1 + 1;
+          bf16x8 rq[kRing1][2], rg[kRing1][2];
+          auto read_rows = [&](auto sc) __attribute__((always_inline)) {
+            constexpr int st = decltype(sc)::value;
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+              rq[st % kRing1][e] = row_operand<kD>(qt, 2 * half + e, st, lane);
+              rg[st % kRing1][e] = row_operand<kD>(gt, 2 * half + e, st, lane);
+            }
+          };
+          static_for<kAhead1>([&](auto sc) { read_rows(sc); });
+          f32x4 sa[2], pa[2];
+#pragma unroll
+          for (int e = 0; e < 2; e++) sa[e] = pa[e] = f32x4{};
+          static_for<T::NS>([&](auto sc) {
+            constexpr int st = decltype(sc)::value;
+            if constexpr (st + kAhead1 < T::NS) read_rows(std::integral_constant<int, st + kAhead1>{});
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+              sa[e] = mfma16(rq[st % kRing1][e], kv[0][st], sa[e]);
+              pa[e] = mfma16(rg[st % kRing1][e], vv[0][st], pa[e]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+          // the first operands of the dK / dV slots, ahead of the softmax and the hand-over
+          constexpr int kAhead2 = 4, kRing2 = kAhead2 + 1;
+          bf16x8 cg[kRing2], cq[kRing2];
+          auto read_cols = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, t = i / ND, db = i % ND;
+            cg[i % kRing2] = col_operand<kD>(gt, 32 * t, 16 * (ND * half + db), lane);
+            cq[i % kRing2] = col_operand<kD>(qt, 32 * t, 16 * (ND * half + db), lane);
+          };
+          static_for<kAhead2>([&](auto ic) { read_cols(ic); });
+          {
+            const int kp = kw0 + i16;
+            float pf[2][4], df[2][4];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+              // register r: query 32 half + 8 g + 4 e + r of the block
+              const f32x4 ls = *reinterpret_cast<const f32x4*>(nlse + 32 * half + 8 * g + 4 * e);
+              const f32x4 dl = *reinterpret_cast<const f32x4*>(ndel + 32 * half + 8 * g + 4 * e);
+#pragma unroll
+              for (int r = 0; r < 4; r++) {
+                float x = fmaf(sa[e][r], c2, ls[r]);
+                if (diag) x = kp <= tok0 + 32 * half + 8 * g + 4 * e + r ? x : -INFINITY;
+                pf[e][r] = fast_exp2(x);
+                df[e][r] = pf[e][r] * (pa[e][r] + dl[r]);
+              }
+            }
+            bf16x8* mine = hand + (kgroup * 2 + half) * 2 * 64 + lane;
+            const bf16x8 ds = pack8(df[0], df[1]);
+            mine[0] = pack8(pf[0], pf[1]);
+            mine[64] = ds;
+            if constexpr (kStoreDs) {
+              // dS of the 32-query half, lane l: key l % 16, queries 8 (l / 16) .. +7: one
+              // whole 1 KiB line, streaming buffer store from the stage's uniform base
+              __builtin_amdgcn_raw_buffer_store_b128(
+                  __builtin_bit_cast(i32x4_m16, ds),
+                  __builtin_amdgcn_make_buffer_rsrc(ds_stage, 0, m16_ds_head_bytes(kD) / kM16Waves, 0x00020000),
+                  half * 1024 + 16 * lane, 0, 2 /* non-temporal */);
+            }
+          }
+          // Both waves of a pair have written. Only LDS is waited for: the next
+          // stage's copies and the dS stores stay in flight.
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          static_for<2 * ND>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, t = i / ND, db = i % ND;
+            if constexpr (i + kAhead2 < 2 * ND) read_cols(std::integral_constant<int, i + kAhead2>{});
+            if constexpr (db == 0) {
+              pT[0] = hand[(kgroup * 2 + t) * 2 * 64 + lane];
+              dT[0] = hand[(kgroup * 2 + t) * 2 * 64 + 64 + lane];
+            }
+            dv[0][db] = mfma16(pT[0], cg[i % kRing2], dv[0][db]);
+            dk[0][db] = mfma16(dT[0], cq[i % kRing2], dk[0][db]);
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        } else {
         // The stage is one fixed sequence of slots, each fenced: per query-block
         // pair t, the S / dP slots (e = 0, 1; k-steps s) and then the dV / dK
         // slots (head-dim blocks db). Every slot takes two operands from LDS
@@ -1191,7 +1291,6 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
         f32x4 sa[KB], pa[KB];
         f32x4 ls, dl;                                  // -lse*log2e, -delta of the block's queries
         float pf[KB][2][4], df[KB][2][4];              // [key block][query block 2t + e][register]
-        bf16x8 pT[KB], dT[KB];                         // queries 32 t + 8 g + 0..7 of key 16 kb + l % 16
         static_for<kSlots>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
           constexpr int t = i / kPT, j = i % kPT;
@@ -1232,15 +1331,6 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
                   pT[kb] = pack8(pf[kb][0], pf[kb][1]);
                   dT[kb] = pack8(df[kb][0], df[kb][1]);
                 }
-                if constexpr (kStoreDs) {
-                  // dS of the 32-query half t, lane l: key l % 16, queries 32 t + 8 (l / 16) .. +7:
-                  // one whole 1 KiB line, streaming buffer store from the stage's uniform base
-                  static_assert(KB == 1, "one 16-key block per wave");
-                  __builtin_amdgcn_raw_buffer_store_b128(
-                      __builtin_bit_cast(i32x4_m16, dT[0]),
-                      __builtin_amdgcn_make_buffer_rsrc(ds_stage, 0, m16_ds_head_bytes(kD) / kM16Waves, 0x00020000),
-                      t * 1024 + 16 * lane, 0, 2 /* non-temporal */);
-                }
               }
             }
           } else {
@@ -1253,6 +1343,9 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
           }
           __builtin_amdgcn_sched_barrier(0);
         });
+              }
+      } else if constexpr (kShare) {
+        asm volatile("s_barrier" ::: "memory");  // the hand-over's
       }
       wait_dma();  // stage sidx + 1 has landed
       __syncthreads();
@@ -1263,7 +1356,7 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
       // hoisted out of the tile loop
       int el = lane;
       asm volatile("" : "+v"(el));
-      const int i16 = el & 15, g = el >> 4;
+      const int g = el >> 4, col0 = 16 * ND * half + (el & 15);  // the wave's first column, this lane's
       const int slot = item[DK_SLOT];  // -1 for a pair: its tiles are never split
       if (slot >= 0) {  // split tile: fp32 partial [kKeys][kD] for dK (already scaled) then dV
         float* pk = a.ws + static_cast<int64_t>(slot) * 2 * kKeys * kD;
@@ -1272,27 +1365,27 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll
           for (int r = 0; r < 4; r++) {
-            const int key = kWaveKeys * wave + 16 * kb + 4 * g + r;
+            const int key = kWaveKeys * kgroup + 16 * kb + 4 * g + r;
 #pragma unroll
-            for (int db = 0; db < T::ND; db++) {
-              pk[key * kD + 16 * db + i16] = dk[kb][db][r] * a.scale;
-              pv[key * kD + 16 * db + i16] = dv[kb][db][r];
+            for (int db = 0; db < ND; db++) {
+              pk[key * kD + 16 * db + col0] = dk[kb][db][r] * a.scale;
+              pv[key * kD + 16 * db + col0] = dv[kb][db][r];
             }
           }
       } else if (prefix && a.acc_prefix) {
         // a tensor's old values are all read before the first is written (reads
         // behind writes that may alias them would wait row by row)
-        auto add_rows = [&](float* base, const f32x4 (&acc)[KB][T::ND], float mul) __attribute__((always_inline)) {
+        auto add_rows = [&](float* base, const f32x4 (&acc)[KB][ND], float mul) __attribute__((always_inline)) {
 #pragma clang fp contract(off)
-          float old[KB][4][T::ND];
+          float old[KB][4][ND];
 #pragma unroll
           for (int kb = 0; kb < KB; kb++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
               const int key = min(kw0 + 16 * kb + 4 * g + r, seg_len - 1);
-              const float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
+              const float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + col0;
 #pragma unroll
-              for (int db = 0; db < T::ND; db++) old[kb][r][db] = row[16 * db];
+              for (int db = 0; db < ND; db++) old[kb][r][db] = row[16 * db];
             }
 #pragma unroll
           for (int kb = 0; kb < KB; kb++)
@@ -1300,9 +1393,9 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
             for (int r = 0; r < 4; r++) {
               const int key = kw0 + 16 * kb + 4 * g + r;
               if (key >= seg_len) continue;
-              float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
+              float* row = base + static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + col0;
 #pragma unroll
-              for (int db = 0; db < T::ND; db++) row[16 * db] = old[kb][r][db] + acc[kb][db][r] * mul;
+              for (int db = 0; db < ND; db++) row[16 * db] = old[kb][r][db] + acc[kb][db][r] * mul;
             }
         };
         add_rows(static_cast<float*>(a.dpk), dk, a.scale);
@@ -1316,9 +1409,9 @@ __global__ __launch_bounds__(256) void m16_dkdv(KernelArgs a) {
           for (int r = 0; r < 4; r++) {
             const int key = kw0 + 16 * kb + 4 * g + r;
             if (key >= seg_len) continue;
-            const int64_t off = static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + i16;
+            const int64_t off = static_cast<int64_t>(seg_row0 + key) * kstride + kvh * kD + col0;
 #pragma unroll
-            for (int db = 0; db < T::ND; db++) {
+            for (int db = 0; db < ND; db++) {
               dkd[off + 16 * db] = static_cast<bf16>(dk[kb][db][r] * a.scale);
               dvd[off + 16 * db] = static_cast<bf16>(dv[kb][db][r]);
             }
@@ -1404,13 +1497,13 @@ int launch_dkdv_d(const KernelArgs& a, int n_dkdv, int n_red, hipStream_t s) {
   if (n_dkdv > 0) {
     const bool st = strided_rows<kD>(a), ds = kD == 256 && a.ds != nullptr;
     if (st && ds)
-      hipLaunchKernelGGL((m16_dkdv<kD, true, kD == 256>), dim3(n_dkdv), dim3(64 * kM16Waves), 0, s, a);
+      hipLaunchKernelGGL((m16_dkdv<kD, true, kD == 256>), dim3(n_dkdv), dim3(64 * m16_dkdv_waves(kD)), 0, s, a);
     else if (st)
-      hipLaunchKernelGGL((m16_dkdv<kD, true, false>), dim3(n_dkdv), dim3(64 * kM16Waves), 0, s, a);
+      hipLaunchKernelGGL((m16_dkdv<kD, true, false>), dim3(n_dkdv), dim3(64 * m16_dkdv_waves(kD)), 0, s, a);
     else if (ds)
-      hipLaunchKernelGGL((m16_dkdv<kD, false, kD == 256>), dim3(n_dkdv), dim3(64 * kM16Waves), 0, s, a);
+      hipLaunchKernelGGL((m16_dkdv<kD, false, kD == 256>), dim3(n_dkdv), dim3(64 * m16_dkdv_waves(kD)), 0, s, a);
     else
-      hipLaunchKernelGGL((m16_dkdv<kD, false, false>), dim3(n_dkdv), dim3(64 * kM16Waves), 0, s, a);
+      hipLaunchKernelGGL((m16_dkdv<kD, false, false>), dim3(n_dkdv), dim3(64 * m16_dkdv_waves(kD)), 0, s, a);
     if (hipGetLastError() != hipSuccess) return 4;
   }
   if (n_red > 0) {
