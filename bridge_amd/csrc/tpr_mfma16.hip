@@ -1042,7 +1042,8 @@ __global__ __launch_bounds__(64 * m16_dkdv_waves(kD)) void m16_dkdv(KernelArgs a
   // and dV, and they hand each other P and dS through LDS. One wave for 16 keys
   // (one a SIMD) waited on its own LDS reads, 128 KB a stage at 35 to 51 bytes a
   // cycle beside 2048 cycles of MFMA; now the unit's 512 KB of LDS reads a stage
-  // bound it. A layer pass at prefix 4096 + 4 x 4096, GQA 8/2: 3386 -> 3300 us.
+  // bound it. A layer pass at prefix 4096 + 4 x 4096, GQA 8/2: 3385 -> 3177 us,
+  // its dK/dV 2217 -> 1914.
   // (Four waves, two sharing 32 keys: half the LDS reads, but one wave a SIMD
   // again, 3584 us.)
   constexpr bool kShare = kD == 256;
