@@ -206,16 +206,19 @@ def _check_accumulators(accumulators, prefix_k) -> Tuple[torch.Tensor, torch.Ten
 
 
 def _workspace(meta, q, k, budget, ws, masked=False):
-    """(plan, workspace, its bytes) of the backward. Where the workspace cannot
-    be allocated the backward runs without its parts, and a plan with a dS
-    store falls back to the plan without one (a few MB), which gives the same
-    gradients with a slower dQ."""
+    """(plan, workspace, its bytes) of the backward. A workspace given by the
+    caller counts with the bytes it has: the library refuses less than
+    ``plan.bwd_min_bytes`` and runs the parts only in ``plan.workspace_bytes``.
+    Where the workspace cannot be allocated the backward runs without its
+    parts, and a plan with a dS store falls back to the plan without one (a few
+    MB), which gives the same gradients with a slower dQ."""
     def empty(size):
         return torch.empty(size, dtype=torch.uint8, device=q.device) if size else None
 
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=budget, masked=masked)
     if ws is not None:
-        return plan, ws, plan.workspace_bytes
+        behind = ws.untyped_storage().nbytes() - ws.storage_offset() * ws.element_size()
+        return plan, ws, min(ws.numel() * ws.element_size(), behind)
     plans = [plan]
     if plan.dq_from_ds:
         plans.append(None)  # the plan without a store, built only if needed
@@ -362,8 +365,10 @@ def prefix_attention_backward(q, k, v, prefix_k, prefix_v, out, lse, dout, meta:
     prefix_k into which the prefix gradients are added (and returned).
     ``ds_store_budget`` (bytes; None = the library default) or
     ``recompute_dq=True`` (= budget 0) select the plan (TPRPrefixMeta.plan);
-    with a dS store the dQ phase reads what the dK/dV phase wrote, and a
-    ``workspace`` given in ``buffers`` must be of that plan's size.
+    with a dS store the dQ phase reads what the dK/dV phase wrote. A
+    ``workspace`` given in ``buffers`` has at least that plan's
+    ``bwd_min_bytes``; with less than its ``workspace_bytes`` the backward runs
+    without its parts.
     ``attention_mask``: the forward's physical key mask, if it had one."""
     scale = validate(q, k, v, prefix_k, prefix_v, meta, softmax_scale)
     mask = check_mask(attention_mask, q, meta)

@@ -11,9 +11,7 @@ delta from the rounded output, and dP - delta cancels where a row has few keys
 
 from __future__ import annotations
 
-import dataclasses
 import math
-from unittest import mock
 
 import pytest
 import torch
@@ -54,15 +52,16 @@ def test_dkdv_parts_match_oracle_and_whole_items(name, d, recompute, relay, cuda
           f"{int(plan.host[N_KPART + 4])} slots", flush=True)
     out, lse = prefix_attention_forward(q, k, v, pk, pv, meta, scale)
 
-    def backward(sized):
+    def backward(size):
         acc = tuple(torch.full(pk.shape, 0.25, dtype=torch.float32, device=cuda_device) for _ in range(2)) if relay else None
-        ws = torch.empty(sized.workspace_bytes, dtype=torch.uint8, device=cuda_device)
-        with mock.patch.object(type(meta), "plan", return_value=sized):
-            return prefix_attention_backward(q, k, v, pk, pv, out, lse, dout, meta, scale, recompute_dq=recompute,
-                                             prefix_grad_accumulators=acc, buffers={"workspace": ws})
+        room = torch.full((size + (1 << 20),), 0x5a, dtype=torch.uint8, device=cuda_device)
+        grads = prefix_attention_backward(q, k, v, pk, pv, out, lse, dout, meta, scale, recompute_dq=recompute,
+                                          prefix_grad_accumulators=acc, buffers={"workspace": room[:size]})
+        assert bool((room[size:] == 0x5a).all()), "written past the workspace"
+        return grads
 
-    parts, again = backward(plan), backward(plan)
-    whole = backward(dataclasses.replace(plan, workspace_bytes=plan.bwd_min_bytes))
+    parts, again = backward(plan.workspace_bytes), backward(plan.workspace_bytes)
+    whole = backward(plan.bwd_min_bytes)
     torch.cuda.synchronize()
     _, _, ref = oracle(meta, q, k, v, pk, pv, dout, scale)
     for i, label in enumerate(("dq", "dk", "dv", "dprefix_k", "dprefix_v")):
