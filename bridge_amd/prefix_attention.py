@@ -205,6 +205,22 @@ def _check_accumulators(accumulators, prefix_k) -> Tuple[torch.Tensor, torch.Ten
     return accumulators[0], accumulators[1]
 
 
+def _allocate(plan, device, must):
+    """(workspace, its bytes) for a plan's backward: the full size, or the least
+    where that does not fit. Where neither does: None, or with ``must`` the
+    allocator's error. The error is never held: a caught exception kept in a
+    local would keep the callers' frames, and every tensor in them, until the
+    cyclic collector runs."""
+    least = plan.workspace_bytes if plan.bwd_min_bytes is None else plan.bwd_min_bytes
+    for size in sorted({plan.workspace_bytes, least}, reverse=True):
+        try:
+            return torch.empty(size, dtype=torch.uint8, device=device) if size else None, size
+        except torch.OutOfMemoryError:
+            if must and size == least:
+                raise
+    return None
+
+
 def _workspace(meta, q, k, budget, ws, masked=False):
     """(plan, workspace, its bytes) of the backward. A workspace given by the
     caller counts with the bytes it has: the library refuses less than
@@ -212,25 +228,15 @@ def _workspace(meta, q, k, budget, ws, masked=False):
     Where the workspace cannot be allocated the backward runs without its
     parts, and a plan with a dS store falls back to the plan without one (a few
     MB), which gives the same gradients with a slower dQ."""
-    def empty(size):
-        return torch.empty(size, dtype=torch.uint8, device=q.device) if size else None
-
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=budget, masked=masked)
     if ws is not None:
         behind = ws.untyped_storage().nbytes() - ws.storage_offset() * ws.element_size()
         return plan, ws, min(ws.numel() * ws.element_size(), behind)
-    plans = [plan]
-    if plan.dq_from_ds:
-        plans.append(None)  # the plan without a store, built only if needed
-    for p in plans:
-        p = p or meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
-        least = p.workspace_bytes if p.bwd_min_bytes is None else p.bwd_min_bytes
-        for size in sorted({p.workspace_bytes, least}, reverse=True):
-            try:
-                return p, empty(size), size
-            except torch.OutOfMemoryError as exc:
-                error = exc
-    raise error
+    got = _allocate(plan, q.device, must=not plan.dq_from_ds)
+    if got is None:
+        plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
+        got = _allocate(plan, q.device, must=True)
+    return plan, *got
 
 
 def _backward(q, k, v, prefix_k, prefix_v, out, lse, dout, meta, scale, *, phases=None, buffers=None,
