@@ -19,10 +19,11 @@
 // us): fp32, prefix 1024 + 2 x 1024, GQA 32/8, d128: 1222 / 4094 / 1260 ->
 // 403 / 930 / 590 (128 TFLOP/s in the forward, of 154); fp32, prefix 512 + 2 x
 // 512, 4 heads, d64: 375 / 485 / 317 -> 26 / 47 / 33; bf16, prefix 1024 + 3 x
-// 1024, GQA 32/8, d96: 1276 / 6116 / 1703 -> 165 / 441 / 187; bf16 under a
-// causal mask with padding, 1024 + 2048, GQA 32/8, d128: 2409 / 4707 / 2590 ->
-// 204 / 662 / 264. What is left in bf16 is the serial chain product - exp -
-// split - product of the one wave a SIMD holds in dK/dV.
+// 1024, GQA 32/8, d96: 1276 / 6116 / 1703 -> 165 / 441 / 187 (before split3
+// kept its terms nonzero); bf16 under a causal mask with padding, 1024 + 2048,
+// GQA 32/8, d128: 2409 / 4707 / 2590 -> 241 / 740 / 298. What is left in bf16
+// is the serial chain product - exp - split - product of the one wave a SIMD
+// holds in dK/dV.
 //
 // A wave owns 32 stationary rows -- queries of one head in the forward and dQ,
 // keys of one KV head in dK/dV -- and streams 32-row tiles of the other side
@@ -144,18 +145,31 @@ __device__ __forceinline__ f32x16 row_product_reload(const char* tile, const ele
   return s;
 }
 
-// x = hi + mid + lo exactly (up to underflow), each a bf16: the top 8
-// mantissa bits, the next 8, the last 8. Truncation, not rounding: hi cannot
-// overflow, and an infinite or NaN x gives a NaN sum as the fp32 product
-// would (x is a probability or a dS).
+// Bits whose high half is the bf16 next to x towards 0 (0 for x = +0): the
+// integer below x's bits, cut to bf16, is always smaller than x.
+__device__ __forceinline__ uint32_t below(float x) { return __builtin_elementwise_sub_sat(__float_as_uint(x), 1u); }
+__device__ __forceinline__ float high_half(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
+
+// x = hi + mid + lo exactly (up to underflow), each a bf16 and, for x != 0,
+// each nonzero and of x's sign: hi is the bf16 below x, mid the bf16 below the
+// rest (at most 2^16 units of x's last place), lo what is left (at most 2^8 of
+// them, or a power of two). A zero term would make NaN of a product with an
+// infinite V, dO, K or Q where the fp32 product is infinite; an infinite x
+// ends in lo, behind two finite terms of its sign. (With the terms cut at x's
+// own bits, 1 = 1 + 0 + 0, two VALU instructions less a value: bf16 under a
+// causal mask, 1024 + 2048, GQA 32/8, d128, forward / dK/dV / dQ 223 / 684 /
+// 281 us against 241 / 740 / 298.) kSigned: x may be -0, which below() does
+// not take.
+template <bool kSigned>
 __device__ __forceinline__ void split3(const float (&x)[8], bf16x8& hi, bf16x8& mid, bf16x8& lo) {
   uint32_t a[4], b[4], c[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const uint32_t x0 = __float_as_uint(x[2 * i]), x1 = __float_as_uint(x[2 * i + 1]);
-    const float r0 = x[2 * i] - __uint_as_float(x0 & 0xffff0000u), r1 = x[2 * i + 1] - __uint_as_float(x1 & 0xffff0000u);
-    const uint32_t u0 = __float_as_uint(r0), u1 = __float_as_uint(r1);
-    const float t0 = r0 - __uint_as_float(u0 & 0xffff0000u), t1 = r1 - __uint_as_float(u1 & 0xffff0000u);
+    const float y0 = kSigned ? x[2 * i] + 0.f : x[2 * i], y1 = kSigned ? x[2 * i + 1] + 0.f : x[2 * i + 1];
+    const uint32_t x0 = below(y0), x1 = below(y1);
+    const float r0 = y0 - high_half(x0), r1 = y1 - high_half(x1);
+    const uint32_t u0 = below(r0), u1 = below(r1);
+    const float t0 = r0 - high_half(u0), t1 = r1 - high_half(u1);
     a[i] = __builtin_amdgcn_perm(x1, x0, 0x07060302u);  // the high halves of the two words
     b[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
     c[i] = __builtin_amdgcn_perm(__float_as_uint(t1), __float_as_uint(t0), 0x07060302u);
@@ -169,8 +183,9 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 // acc[db] += (tile columns)^T x: acc rows are output columns (out_col), acc
 // columns the wave's stationary rows; x[r] belongs to tile row
-// 16 (r / 8) + 8 h + r % 8. kNB column blocks from block db0 on.
-template <int kNB>
+// 16 (r / 8) + 8 h + r % 8. kNB column blocks from block db0 on. kSigned: x is
+// not a probability (split3).
+template <bool kSigned, int kNB>
 __device__ __forceinline__ void col_product(const char* tile, const f32x16& x, f32x16 (&acc)[kNB], int db0, int lane) {
   const int n = lane & 31, h = lane >> 5;
   if constexpr (kF32) {
@@ -204,7 +219,7 @@ __device__ __forceinline__ void col_product(const char* tile, const f32x16& x, f
 #pragma unroll
       for (int e = 0; e < 8; e++) p[e] = x[8 * c + e];
       bf16x8 hi, mid, lo;
-      split3(p, hi, mid, lo);
+      split3<kSigned>(p, hi, mid, lo);
       const int row = 16 * c + 8 * h + (i >> 2);
 #pragma unroll
       for (int db = 0; db < kNB; db++) {
@@ -267,7 +282,8 @@ __device__ __forceinline__ f32x4 load4f(const float* p) {
 // ---- staging --------------------------------------------------------------
 // One 32-row tile of a [*, heads, d] tensor, copied by kT threads: rows from
 // `base` (head offset applied), `stride` elements apart; rows at or beyond
-// `rows` (>= 1) re-read the last one, columns at or beyond d are 0.
+// `rows` (>= 1) and columns at or beyond d are 0 (a copy of the last row in
+// their place would multiply its infinities by a probability of 0).
 template <int kT>
 struct TileRegs { f32x4 r[kRows * kChunks / kT]; };
 
@@ -299,8 +315,10 @@ __device__ __forceinline__ void fetch_tile(TileRegs<kT>& t, const elem* base, in
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < kPasses; i++)
-      t.r[i] = load_chunk(reinterpret_cast<const elem*>(src + (min(row + kStep * i, rows - 1) * row_bytes + col)));
+    for (int i = 0; i < kPasses; i++) {
+      const f32x4 x = load_chunk(reinterpret_cast<const elem*>(src + (min(row + kStep * i, rows - 1) * row_bytes + col)));
+      t.r[i] = row + kStep * i < rows ? x : f32x4{};
+    }
   }
   if (!in) {
 #pragma unroll
@@ -323,6 +341,10 @@ __device__ __forceinline__ void copy_tile(char* tile, const elem* base, int64_t 
 #pragma unroll
     for (int i = 0; i < kAtOnce; i++)
       r[i] = load_chunk(reinterpret_cast<const elem*>(src + (min(row + kStep * (i0 + i), rows - 1) * row_bytes + col)));
+    if (rows < kRows) {
+#pragma unroll
+      for (int i = 0; i < kAtOnce; i++) r[i] = row + kStep * (i0 + i) < rows ? r[i] : f32x4{};
+    }
 #pragma unroll
     for (int i = 0; i < kAtOnce; i++)
       *reinterpret_cast<f32x4*>(tile + lds_off(row + kStep * (i0 + i), c)) = in ? r[i] : f32x4{};
@@ -668,7 +690,7 @@ __global__ __launch_bounds__(Run<kSplit>::kT, Run<kSplit>::kMinWaves) void gen_f
 #pragma unroll
       for (int r = 0; r < w; r++) x[r] += x[r + w];
     l += x[0];
-    col_product<kDB>(vt, s, o, 0, q.lane);
+    col_product<false>(vt, s, o, 0, q.lane);
   });
   l = wave_sum32(l);
 
@@ -751,7 +773,7 @@ __global__ __launch_bounds__(Run<kSplit>::kT, Run<kSplit>::kMinWaves) void gen_d
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = vis >> r & 1 ? s[r] : 0.f;
     }
-    col_product<kDB>(kt, s, dq, 0, q.lane);
+    col_product<true>(kt, s, dq, 0, q.lane);
   });
 
   elem* out = static_cast<elem*>(a.dq);
@@ -856,6 +878,7 @@ __global__ __launch_bounds__(64 * kQParts) void gen_dkdv(KernelArgs a) {
     if constexpr (kBoth) fetch_g(rg, cur, x);
     const int64_t at = static_cast<int64_t>(head) * a.total_q + cur.row + min(n, cur.toks - 1);
     st = h == 0 ? a.lse_in[at] * kLog2e : a.delta[at];
+    st = n < cur.toks ? st : 0.f;  // rows past the end: p is 0, and dS = p (dP - delta) with it
     if constexpr (kMask) {
       const uint8_t* mrow = a.mask + static_cast<int64_t>(cur.row) * a.mask_rs + cur.col + kp;
       if (cur.toks == kRows) {
@@ -931,8 +954,8 @@ __global__ __launch_bounds__(64 * kQParts) void gen_dkdv(KernelArgs a) {
         dp[r] = p * (dp[r] - de[e >> 2][e & 3]);
       }
     }
-    col_product<kOutB>(gt, s, dv, db0, lane);
-    col_product<kOutB>(qt, dp, dk, db0, lane);
+    col_product<false>(gt, s, dv, db0, lane);
+    col_product<true>(qt, dp, dk, db0, lane);
   }
 
   auto finish = [&](const f32x16 (&acc)[kOutB], float mul, void* prefix_out, void* suffix_out) __attribute__((always_inline)) {
