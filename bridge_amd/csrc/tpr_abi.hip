@@ -402,9 +402,13 @@ int bwd_phases(const TprBwdParams* p, int phases, void* stream, void* workspace,
   }
   const bool fp32 = ph[PF_DTYPE] == TPR_DTYPE_FP32;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int n_dkdv = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) ? ph[kparts ? PF_N_KPART : PF_N_DKDV] : 0;
-  // 0 on the general path
-  const int n_red = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[kparts ? PF_N_KRED : PF_N_RED] : 0;
+  const bool tiles = (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_TILES)) != 0;
+  const int n_dkdv = tiles ? ph[kparts ? PF_N_KPART : PF_N_DKDV] : 0;
+  // The parts' partials are summed by the call that wrote them, so that a
+  // reduction enqueued separately does not depend on that call's workspace
+  // size. (A plan has parts only where its whole items leave no partials.)
+  const int n_red = kparts ? (tiles ? ph[PF_N_KRED] : 0)
+                           : (phases & (TPR_BWD_DKDV | TPR_BWD_DKDV_REDUCE)) ? ph[PF_N_RED] : 0;  // 0 on the general path
   // dQ work items: the forward's, or a dS-store plan's own list
   const int n_dq = (phases & TPR_BWD_DQ) ? (ph[PF_N_DQS] > 0 ? ph[PF_N_DQS] : ph[PF_N_FWD]) : 0;
   if (phases & TPR_BWD_DELTA)

@@ -197,7 +197,7 @@ typedef struct TprBwdParams {
   void* dprefix_k;
   void* dprefix_v;
   void* workspace;        /* 256-byte aligned */
-  size_t workspace_bytes; /* >= tpr_attn_bwd_workspace_bytes(plan_host) */
+  size_t workspace_bytes; /* >= tpr_attn_bwd_min_workspace_bytes(plan_host) */
   /* row strides of q, k and v, as in TprFwdParams (0 = packed); the
    * gradients dq, dk, dv are written packed */
   int64_t q_row_stride;
@@ -220,15 +220,15 @@ const char* tpr_attn_last_error(void);
 int tpr_attn_plan(const TprTreeDesc* tree, int32_t* plan, int64_t capacity_words,
                   int64_t* words_needed);
 
-/* Bytes of workspace the backward needs for this plan (fp32 statistics and
- * partial sums, and the dS store of a plan that has one). */
+/* Bytes of workspace the backward uses for this plan (fp32 statistics and
+ * partial sums, the dS store of a plan that has one, and the parts' slots). */
 size_t tpr_attn_bwd_workspace_bytes(const int32_t* plan_host);
 
 /* The least the backward runs with. Where rows or key tiles are too few or too
  * uneven to fill the GPU, a plan also cuts dQ along the keys and dK/dV along
  * the queries over more workgroups; with less than
  * tpr_attn_bwd_workspace_bytes() those parts do not run (the sums' order, and
- * so the last bits, differ). All phases of one backward must be given the same
+ * so the last bits, differ). Each phase decides by its own call's
  * workspace_bytes. */
 size_t tpr_attn_bwd_min_workspace_bytes(const int32_t* plan_host);
 
@@ -260,7 +260,8 @@ int tpr_attn_bwd(const TprBwdParams* params, void* stream);
 #define TPR_BWD_DELTA 1        /* delta = rowsum(dout * out), fp32 [Hq, Tq] */
 #define TPR_BWD_DKDV 2         /* dk, dv, dprefix_k, dprefix_v */
 #define TPR_BWD_DQ 4           /* dq */
-#define TPR_BWD_DKDV_TILES 8   /* dK/dV tiles; split prefix tiles leave fp32 partials in the workspace */
+#define TPR_BWD_DKDV_TILES 8   /* dK/dV tiles; split prefix tiles leave fp32 partials in the workspace
+                                  (parts of tiles are summed in this step) */
 #define TPR_BWD_DKDV_REDUCE 16 /* ordered sum of those partials into dprefix_k / dprefix_v */
 int tpr_attn_bwd_phases(const TprBwdParams* params, int phases, void* stream);
 

@@ -76,3 +76,37 @@ def test_dkdv_parts_match_oracle_and_whole_items(name, d, recompute, relay, cuda
         assert rel_l2(p, w) <= ULP, label
         err = (p - w).norm(dim=1) / w.norm(dim=1).clamp_min(1e-2 * w.norm() / math.sqrt(len(w)))
         assert err.max().item() <= ULP, label
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("tiles_full", [True, False], ids=["tiles_full", "tiles_least"])
+def test_separate_steps_do_not_depend_on_each_others_workspace(tiles_full, d, cuda_device):
+    """The tiles step and the reduction step, enqueued separately with the full
+    workspace for one and the least for the other: dK, dV and dQ are those of one
+    call with the size that the step which writes them was given, bit for bit."""
+    from bridge_amd import _lib, prefix_attention_backward, prefix_attention_forward
+    meta, hq, hkv, scale = _metas()["ragged"], 6, 2, 1.0 / math.sqrt(d)
+    plan = meta.plan(hq, hkv, d, torch.bfloat16, cuda_device)
+    assert plan.host[N_KPART] > 0
+    q, k, v, pk, pv, dout = make_inputs(meta, hq, hkv, d, torch.bfloat16, seed=5, device=cuda_device)
+    out, lse = prefix_attention_forward(q, k, v, pk, pv, meta, scale)
+    size = {True: plan.workspace_bytes, False: plan.bwd_min_bytes}
+    print(f"[dK/dV steps d{d} tiles_full={tiles_full}]", flush=True)
+
+    def backward(room, full, **more):
+        return prefix_attention_backward(q, k, v, pk, pv, out, lse, dout, meta, scale,
+                                         buffers={"workspace": room[:size[full]], **more.pop("buffers", {})}, **more)
+
+    def room():
+        return torch.full((plan.workspace_bytes,), 0xff, dtype=torch.uint8, device=cuda_device)  # floats read as NaN
+
+    one = {full: backward(room(), full) for full in (True, False)}
+    names = ("dq", "dk", "dv", "dprefix_k", "dprefix_v")
+    mine = {n: torch.full_like(t, math.nan) for n, t in zip(names, one[True])}
+    ws, mine["delta"] = room(), torch.empty_like(lse)
+    for phase, full in ((_lib.TPR_BWD_DELTA, not tiles_full), (_lib.TPR_BWD_DKDV_TILES, tiles_full),
+                        (_lib.TPR_BWD_DKDV_REDUCE, not tiles_full), (_lib.TPR_BWD_DQ, tiles_full)):
+        backward(ws, full, phases=phase, buffers=mine)
+    torch.cuda.synchronize()
+    for name, want in zip(names, one[tiles_full]):
+        assert torch.equal(mine[name], want), name
