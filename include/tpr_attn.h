@@ -267,13 +267,15 @@ int tpr_attn_bwd_phases(const TprBwdParams* params, int phases, void* stream);
 
 /* Allocation-free backward. No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc). Same as tpr_attn_bwd, except
- * that params->workspace / workspace_bytes are ignored: the workspace is the
- * library's static device scratch array, one per GPU, of
- * tpr_attn_bwd_noalloc_max_workspace_bytes() bytes (64 MiB), held from the
+ * serving loops, harnesses that forbid hipMalloc). Same as tpr_attn_bwd with a
+ * workspace of tpr_attn_bwd_noalloc_max_workspace_bytes() bytes (64 MiB),
+ * except that params->workspace / workspace_bytes are ignored: the workspace is
+ * the library's static device scratch array, one per GPU, held from the
  * library's first use on a GPU until the process ends. A plan whose
- * tpr_attn_bwd_workspace_bytes() exceeds that is rejected with
- * TPR_ERR_UNSUPPORTED. The call allocates and frees nothing; the scratch
+ * tpr_attn_bwd_min_workspace_bytes() exceeds that is rejected with
+ * TPR_ERR_UNSUPPORTED; parts of a plan that do not fit beside it do not run
+ * (the last bits differ from tpr_attn_bwd with the plan's full workspace). The
+ * call allocates and frees nothing; the scratch
  * address is looked up once per device (with that device current) on the
  * first call there, which must not be under stream capture (a capturing
  * first call is refused with TPR_ERR_INVALID_ARGUMENT): make one call per

@@ -54,6 +54,51 @@ def test_noalloc_rejects_a_plan_beyond_its_scratch_before_any_launch():
     assert b"static scratch" in lib.tpr_attn_last_error()
 
 
+def _plan_with_parts_beyond_the_scratch(device):
+    """The least workspace fits the static scratch, the parts beside it do not."""
+    meta = TPRPrefixMeta.shared_prefix(15000, [64])
+    return meta, meta.plan(32, 8, 128, torch.bfloat16, device)
+
+
+def test_noalloc_takes_a_plan_whose_least_workspace_fits():
+    """Refused is what cannot run; a plan that can run without its parts passes
+    the size check (what stops it here is the missing tensors or GPU)."""
+    lib = _lib.load()
+    _, plan = _plan_with_parts_beyond_the_scratch(torch.device("cpu"))
+    assert plan.bwd_min_bytes <= lib.tpr_attn_bwd_noalloc_max_workspace_bytes() < plan.workspace_bytes
+    b = _lib.TprBwdParams()
+    b.abi_version = _lib.ABI_VERSION
+    b.softmax_scale = 0.1
+    b.plan_host = b.plan_device = plan.host.data_ptr()
+    status = lib.tpr_attn_bwd_noalloc(ctypes.byref(b), None)
+    assert status not in (0, _lib.TPR_ERR_UNSUPPORTED, _lib.TPR_ERR_BUFFER_TOO_SMALL)
+
+
+@pytest.mark.gpu
+def test_noalloc_runs_as_a_workspace_of_the_scratch_size(cuda_device):
+    """Bit for bit tpr_attn_bwd with 64 MiB of workspace, in which the parts do
+    not run."""
+    lib = _lib.load()
+    stream = ctypes.c_void_p(torch.cuda.current_stream(cuda_device).cuda_stream)
+    meta, plan = _plan_with_parts_beyond_the_scratch(cuda_device)
+    size = lib.tpr_attn_bwd_noalloc_max_workspace_bytes()
+    assert plan.bwd_min_bytes <= size < plan.workspace_bytes
+    q, k, v, pk, pv, dout = make_inputs(meta, 32, 8, 128, torch.bfloat16, seed=7, device=cuda_device)
+    scale = 1.0 / math.sqrt(128)
+    out, lse = prefix_attention_forward(q, k, v, pk, pv, meta, scale)
+    tensors = (q, k, v, pk, pv, out, lse, dout)
+    ws = torch.empty(size, dtype=torch.uint8, device=cuda_device)
+    ref, mine = _fresh_outputs(q, k, v, pk, pv, lse), _fresh_outputs(q, k, v, pk, pv, lse)
+    print(f"[noalloc parts] least {plan.bwd_min_bytes} full {plan.workspace_bytes}", flush=True)
+    p = _bwd_params(plan, scale, tensors, ref, ws)
+    _lib.check(lib.tpr_attn_bwd(ctypes.byref(p), stream), "tpr_attn_bwd")
+    p = _bwd_params(plan, scale, tensors, mine, None)
+    _lib.check(lib.tpr_attn_bwd_noalloc(ctypes.byref(p), stream), "tpr_attn_bwd_noalloc")
+    torch.cuda.synchronize()
+    for label, a, b in zip(("delta", "dq", "dk", "dv", "dprefix_k", "dprefix_v"), mine, ref):
+        assert torch.isfinite(b.float()).all() and torch.equal(a, b), label
+
+
 @pytest.mark.gpu
 def test_noalloc_backward_equals_the_workspace_backward(cuda_device):
     lib = _lib.load()
