@@ -138,17 +138,24 @@ struct Parts {
 // 40: 590, 303, 159, 88, 60; 57. 4096 + 1000: 103, 86, 95, 120, 183; 85.
 // 4096 + 2048: 159, 175, 199, 261, 385; 160 (not cut). d64, 8192 + 512: 136,
 // 80, 62, 63, 69; 59. d256, GQA 8/2: 242, 130, 77, 57, 71; 57.
-Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double fixed, double merge, double per_slot) {
+// `slot_floats`: of a partial slot; a cut whose slots take more than
+// kKeyPartBytes is not made (1200 random workload shapes need at most 176 MiB;
+// without a bound 880 items in two parts each took 234 MB of every forward).
+constexpr int64_t kKeyPartBytes = int64_t{192} << 20;
+Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double fixed, double merge, double per_slot,
+                int slot_floats) {
   Parts out;
   constexpr int kLeastTiles = 3;
   const size_t units = static_cast<size_t>(kPlanCus) * per_cu;
   if (list.empty() || list.size() >= 4 * units) return out;
   int longest = 0;
   for (const QueryItem& q : list) longest = std::max(longest, q.tiles);
+  const int64_t most_slots = kKeyPartBytes / (static_cast<int64_t>(slot_floats) * 4);
   std::vector<int> work;  // one KV head's
+  int slots = 0;          // one KV head's
   auto estimate = [&](int limit) {
     work.clear();
-    int slots = 0;
+    slots = 0;
     for (const QueryItem& q : list) {
       if (q.kvh != 0) continue;
       const int n = (q.tiles + limit - 1) / limit;
@@ -170,7 +177,7 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
     // parts over two rounds of the chip only add slots
     if (l < kLeastTiles || (cut > 2 && work.size() * hkv > 2 * units)) break;
     const double e = estimate(l);
-    if (e < best) {
+    if (e < best && static_cast<int64_t>(slots) * hkv <= most_slots) {
       best = e;
       limit = l;
     }
@@ -637,16 +644,16 @@ static int build_plan(const TprTreeDesc* t, std::vector<int32_t>& plan) {
     }
     const int fwd_per_cu = D == 64 ? 3 : 1, dq_per_cu = D == 64 ? 2 : 1;
     const double slot = D == 128 ? 0.07 : 0.035;
-    fparts = key_parts(fwd_list, Hkv, fwd_per_cu, 4, 4, slot);
+    fparts = key_parts(fwd_list, Hkv, fwd_per_cu, 4, 4, slot, fpart_slot_floats(path, D));
     if (n_dqs > 0) {
       const int tokens = (path == PATH_MFMA ? kDqsTokens : kM16Tokens) * (kM16DqsWaves / gcd_int(G, kM16DqsWaves));
       for (int i = 0; i < n_dqs; i++) {
         const int32_t* w = &dqs_words[4 * i];
         if (w[0] >= 0) dqs_list.push_back({w[0], w[1], w[2], w[3], ds_table[M + w[0]] + suffix_tiles(w, tokens, KT)});
       }
-      qparts = key_parts(dqs_list, Hkv, 1, 3, 2, 0.07);
+      qparts = key_parts(dqs_list, Hkv, 1, 3, 2, 0.07, qpart_slot_floats(path, D, true));
     } else if (path == PATH_MFMA16) {
-      qparts = key_parts(fwd_list, Hkv, dq_per_cu, 4, 4, slot);
+      qparts = key_parts(fwd_list, Hkv, dq_per_cu, 4, 4, slot, qpart_slot_floats(path, D, false));
     }
   }
 

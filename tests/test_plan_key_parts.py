@@ -3,6 +3,7 @@ exactly one part, partial slots used once and summed by one merge, no parts
 where whole items fill the chip -- and the forward workspace's checks."""
 
 import ctypes
+import random
 from collections import defaultdict
 
 import pytest
@@ -106,6 +107,27 @@ def test_parts_only_where_rows_are_few(d, hq, hkv):
     assert counts(100, [64]) == (0, 0)                  # too few tiles to cut
     few = counts(16384, [64])
     assert few[0] >= 64 and few[1] >= 64
+
+
+def test_partial_slots_are_bounded():
+    """At most 192 MiB of partial slots in the forward and in dQ, also where the
+    items (just under four rounds of the chip) would be cut into many."""
+    rng = random.Random(5)
+    shapes = [(40, 8, 128, 60000, [5541]), (16, 2, 256, 40000, [6305]), (32, 8, 128, 32768, [7000]), (32, 8, 64, 60000, [20000])]
+    for _ in range(40):
+        hq, hkv, d = rng.choice([(32, 8, 128), (40, 8, 128), (16, 2, 128), (16, 2, 256), (8, 2, 256), (32, 8, 64)])
+        rows = rng.randrange(400, 1024) * 256 // hq  # 400 to 1023 items of 256 rows
+        shapes.append((hq, hkv, d, rng.randrange(8192, 65536), [rows // 3, rows - rows // 3]))
+    cut = 0
+    for hq, hkv, d, prefix, lens in shapes:
+        for recompute in (False, True):
+            plan = TPRPrefixMeta.shared_prefix(prefix, lens).plan(hq, hkv, d, torch.bfloat16, CPU, recompute_dq=recompute)
+            w = plan.host.tolist()
+            dq_rows = (512 if d == 128 else 256) if plan.dq_from_ds else 128
+            assert plan.fwd_workspace_bytes <= 192 << 20
+            assert w[N_QPART + 4] * dq_rows * d * 4 <= 192 << 20
+            cut += w[N_FPART] > 0
+    assert cut >= 10
 
 
 def test_forward_workspace_checks():
