@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <cstring>
 #include <functional>
+#include <limits>
 #include <numeric>
 #include <vector>
 
@@ -39,25 +40,43 @@ int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // Deal items into per-XCD queues and interleave; pads with empty items
 // (first word -1) so every queue has the same length.
-std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words_per_item, int32_t* count,
+std::vector<int32_t> order_for_xcds(const std::vector<Item>& items, int hkv, int words_per_item, int32_t* count,
                                     bool two_per_cu = false) {
-  std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.work > b.work; });
+  // Most work first, else in the given order: runs of equal work (a tile's KV
+  // heads follow each other) as (-work, first item, items). Sorting the 48-byte
+  // items one by one took half of a small plan's time.
+  struct Run {
+    int64_t neg_work;
+    int first, n;
+  };
+  std::vector<Run> runs;
+  for (int i = 0; i < static_cast<int>(items.size()); i++) {
+    if (runs.empty() || runs.back().neg_work != -items[i].work) runs.push_back({-items[i].work, i, 0});
+    runs.back().n++;
+  }
+  std::sort(runs.begin(), runs.end(), [](const Run& a, const Run& b) {
+    return a.neg_work != b.neg_work ? a.neg_work < b.neg_work : a.first < b.first;
+  });
   std::vector<std::vector<const Item*>> queue(kXcds);
+  for (auto& q : queue) q.reserve(items.size() / kXcds + 1);
   std::vector<int64_t> load(kXcds, 0);
-  for (const Item& it : items) {
-    int best = -1;
-    if (hkv % kXcds == 0) {
-      best = it.kvh % kXcds;
-    } else if (kXcds % hkv == 0) {
-      // head h owns XCDs {h, h + hkv, h + 2*hkv, ...}
-      for (int x = it.kvh; x < kXcds; x += hkv)
-        if (best < 0 || load[x] < load[best]) best = x;
-    } else {
-      for (int x = 0; x < kXcds; x++)
-        if (best < 0 || load[x] < load[best]) best = x;
+  for (const Run& run : runs) {
+    for (int i = run.first; i < run.first + run.n; i++) {
+      const Item& it = items[i];
+      int best = -1;
+      if (hkv % kXcds == 0) {
+        best = it.kvh % kXcds;
+      } else if (kXcds % hkv == 0) {
+        // head h owns XCDs {h, h + hkv, h + 2*hkv, ...}
+        for (int x = it.kvh; x < kXcds; x += hkv)
+          if (best < 0 || load[x] < load[best]) best = x;
+      } else {
+        for (int x = 0; x < kXcds; x++)
+          if (best < 0 || load[x] < load[best]) best = x;
+      }
+      queue[best].push_back(&it);
+      load[best] += it.work;
     }
-    queue[best].push_back(&it);
-    load[best] += it.work;
   }
   // Two workgroups run on a CU at once: when a queue is no longer than its
   // XCD's slots, the CUs' second items run beside the first ones, so the
@@ -68,16 +87,14 @@ std::vector<int32_t> order_for_xcds(std::vector<Item>& items, int hkv, int words
         std::reverse(q.begin() + kPlanCus / kXcds, q.end());
   size_t depth = 0;
   for (auto& q : queue) depth = std::max(depth, q.size());
-  std::vector<int32_t> out;
-  out.reserve(depth * kXcds * words_per_item);
+  std::vector<int32_t> out(depth * kXcds * words_per_item, 0);
+  int32_t* at = out.data();
   for (size_t i = 0; i < depth; i++) {
-    for (int x = 0; x < kXcds; x++) {
-      if (i < queue[x].size()) {
-        out.insert(out.end(), queue[x][i]->words, queue[x][i]->words + words_per_item);
-      } else {
-        out.push_back(-1);
-        out.insert(out.end(), words_per_item - 1, 0);
-      }
+    for (int x = 0; x < kXcds; x++, at += words_per_item) {
+      if (i < queue[x].size())
+        std::memcpy(at, queue[x][i]->words, words_per_item * sizeof(int32_t));
+      else
+        at[0] = -1;
     }
   }
   // drop trailing all-empty rows (cannot happen: the first row is full when any item exists)
@@ -98,14 +115,41 @@ struct QueryItem {
   int32_t leaf, tok, qh, kvh, tiles;
 };
 
+// Largest first. The costs of a plan are small numbers, many of them equal.
+void sort_down(std::vector<int>& costs, int64_t most) {
+  if (most > 8 * static_cast<int64_t>(costs.size()) + 1024) {
+    std::sort(costs.begin(), costs.end(), std::greater<int>());
+    return;
+  }
+  std::vector<int> count(most + 1, 0);
+  for (int c : costs) count[c]++;
+  size_t at = 0;
+  for (int64_t c = most; c >= 0; c--)
+    for (int i = 0; i < count[c]; i++) costs[at++] = static_cast<int>(c);
+}
+
 // Time of one head's workgroup costs (any order) dealt longest first to the
 // first free slot of the XCDs that run that head; every KV head has the same
 // tiles, so one head (or all, where heads share XCDs) stands for the launch.
-int64_t pool_makespan(std::vector<int>& costs, int hkv, int per_cu) {
+//
+// `overhead` comes on top. A result of at least `best` is of no interest: where
+// the largest cost or the even share is that much already, the one that is
+// returned, undealt (most candidates of a plan end here: the planner's time at
+// prefix 8192 + 512, GQA 32/8, d128, 96 -> 67 us together with the sorts by runs
+// and counts; 738 + 3016 + 905, GQA 16/2, 229 -> 93).
+double pool_time(std::vector<int>& costs, int hkv, int per_cu, double overhead, double best) {
   const int copies = hkv % kXcds == 0 ? hkv / kXcds : kXcds % hkv == 0 ? 1 : hkv;
   const int xcds = hkv % kXcds == 0 ? 1 : kXcds % hkv == 0 ? kXcds / hkv : kXcds;
   const size_t slots = static_cast<size_t>(xcds) * (kPlanCus / kXcds) * per_cu;
-  std::sort(costs.begin(), costs.end(), std::greater<int>());
+  int64_t total = 0, most = 0;
+  for (int c : costs) {
+    total += c;
+    most = std::max<int64_t>(most, c);
+  }
+  const double least = std::max(static_cast<double>(most), static_cast<double>(total * copies) / static_cast<double>(slots)) + overhead;
+  if (least >= best) return least;
+  if (costs.size() * copies <= slots) return static_cast<double>(most) + overhead;
+  sort_down(costs, most);
   std::vector<int64_t> ends;
   ends.reserve(slots);
   int64_t end = 0;
@@ -122,7 +166,7 @@ int64_t pool_makespan(std::vector<int>& costs, int hkv, int per_cu) {
         std::push_heap(ends.begin(), ends.end(), std::greater<int64_t>());
       }
     }
-  return end;
+  return static_cast<double>(end) + overhead;
 }
 
 struct Parts {
@@ -153,7 +197,7 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
   const int64_t most_slots = kKeyPartBytes / (static_cast<int64_t>(slot_floats) * 4);
   std::vector<int> work;  // one KV head's
   int slots = 0;          // one KV head's
-  auto estimate = [&](int limit) {
+  auto estimate = [&](int limit, double best) {
     work.clear();
     slots = 0;
     for (const QueryItem& q : list) {
@@ -163,9 +207,9 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
         work.push_back(q.tiles * (p + 1) / n - q.tiles * p / n + static_cast<int>(fixed));
       if (n > 1) slots += n;
     }
-    return static_cast<double>(pool_makespan(work, hkv, per_cu)) + (slots ? merge + per_slot * slots * hkv : 0.0);
+    return pool_time(work, hkv, per_cu, slots ? merge + per_slot * slots * hkv : 0.0, best);
   };
-  const double whole = estimate(longest);
+  const double whole = estimate(longest, std::numeric_limits<double>::infinity());
   // less than this is not worth a second launch: a full chip, or short streams
   int64_t total = 0;
   for (int w : work) total += static_cast<int64_t>(w) * hkv;
@@ -176,7 +220,7 @@ Parts key_parts(const std::vector<QueryItem>& list, int hkv, int per_cu, double 
     const int l = (longest + cut - 1) / cut;
     // parts over two rounds of the chip only add slots
     if (l < kLeastTiles || (cut > 2 && work.size() * hkv > 2 * units)) break;
-    const double e = estimate(l);
+    const double e = estimate(l, best);
     if (e < best && static_cast<int64_t>(slots) * hkv <= most_slots) {
       best = e;
       limit = l;
@@ -228,7 +272,7 @@ Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base
       total += costs.back();
     }
   if (costs.empty()) return out;
-  double best = 0.92 * static_cast<double>(pool_makespan(costs, hkv, per_cu));
+  double best = 0.92 * pool_time(costs, hkv, per_cu, 0.0, std::numeric_limits<double>::infinity());
   // a launch this well balanced already is not worth more partials
   if (static_cast<double>(total) * hkv / units >= best) return out;
   int longest[2] = {1, 1};
@@ -246,7 +290,7 @@ Parts dkdv_parts(const std::vector<DkTile>& tiles, const std::vector<Item>& base
     }
     pieces *= hkv;
     slots *= hkv;
-    return static_cast<double>(pool_makespan(costs, hkv, per_cu)) + (slots ? pass + per_slot * static_cast<double>(slots) : 0.0);
+    return pool_time(costs, hkv, per_cu, slots ? pass + per_slot * static_cast<double>(slots) : 0.0, best);
   };
   int cap[2] = {kDkdvMaxBlocks, kDkdvMaxBlocks};
   bool found = false;
