@@ -1,6 +1,6 @@
 """GPU: physical key masks -- the reference's custom-mask mode
 (rectangular_attention.py:112-122, sparse mode 0: the mask is the only
-visibility rule) -- on the masked SIMT kernels, through the C ABI, against the
+visibility rule) -- on the masked general kernels, through the C ABI, against the
 fp64 oracle (oracle/tpr_oracle.py tree_forward / tree_backward with ``mask``).
 
 Masks are random (about 40% of each row's keys hidden, so rows also see later
@@ -106,7 +106,7 @@ def _check_masked(name, meta, hq, hkv, empty, dtype, d, mask_seed, cuda_device):
 
 def test_causal_mask_on_the_masked_kernels_equals_the_causal_kernels(cuda_device):
     """fp32: the causal mask passed as a physical mask (masked kernels, every
-    suffix key streamed) gives the unmasked SIMT kernels' results."""
+    suffix key streamed) gives the unmasked general kernels' results."""
     from bridge_amd import TPRPrefixMeta, tpr_prefix_attention
     meta = TPRPrefixMeta.shared_prefix(50, [70, 33])
     tree = tree_of(meta)

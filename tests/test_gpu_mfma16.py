@@ -2,7 +2,7 @@
 the C ABI) against the fp64 oracle.
 
 The cases mirror the head_dim-128 MFMA suite (tests/test_gpu_parity.py) and
-the cases the SIMT kernels ran at these sizes before: shared prefixes at GQA
+the cases the vector-ALU kernels ran at these sizes before: shared prefixes at GQA
 ratios 1, 2, 3, 4 and 8 (1, 2 and 4 query heads per forward workgroup), no
 prefix, tile-aligned and ragged lengths, a depth-3 tree, an unused node, empty
 leaves, a 12-level chain as one key run and as 12 separate runs (the run-list

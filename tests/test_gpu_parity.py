@@ -162,7 +162,7 @@ def test_simt_matches_oracle(name, cuda_device):
     meta, hq, hkv, d, dtype = _simt_cases()[name]
     scale = 1.0 / math.sqrt(d)
     q, k, v, pk, pv, dout = make_inputs(meta, hq, hkv, d, dtype, seed=3, device=cuda_device)
-    # bf16 at head_dim 64 and 256 runs on the 16-wide MFMA kernels, the rest on SIMT
+    # bf16 at head_dim 64 and 256 runs on the 16-wide MFMA kernels, the rest on the general kernels
     plan = meta.plan(hq, hkv, d, dtype, cuda_device)
     if dtype == torch.bfloat16 and d in (64, 256):
         assert plan.path == "mfma" and plan.mfma_shape == "16x16x32"

@@ -118,7 +118,7 @@ def test_physical_padding_mask_matches_logical_attention_forward_and_backward(cu
     127, causal mask): output within 6e-3 / 1e-2, gradients of the logical
     rows within 6e-3 / 2e-2, the padding rows' gradients zero, and the fully
     hidden row's output zero -- the reference's assertions. The masked calls
-    run on the masked SIMT kernels, the logical one on the 16x16x32 MFMA
+    run on the masked general kernels, the logical one on the 16x16x32 MFMA
     kernels."""
     from bridge_amd import rectangular_causal_attention
     lq, lkv, hq, hkv, d = 63, 127, 4, 2, 64

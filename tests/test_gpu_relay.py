@@ -6,7 +6,7 @@
   fp32 add per element); dq/dk/dv are those of the ordinary backward; and the
   gradient matches the fp32 oracle -- on the head_dim-128 MFMA path with
   unsplit and with split (reduced) prefix tiles, on the 16-wide MFMA path
-  (head_dim 64, and 256 with split tiles), and on the SIMT paths (fp32, and
+  (head_dim 64, and 256 with split tiles), and on the general kernels (fp32, and
   bf16 at head_dim 96).
 * A DFS through PrefixKVStack with TPRKernelBackend.from_stack relays every
   node's gradient (fp32, summed over two sibling batches for the root) to the
@@ -64,7 +64,7 @@ def test_accumulate_mode_adds_the_prefix_gradient(case, cuda_device):
     elif case == "mfma16_split_d256":  # head_dim 256 with split prefix tiles (partials + reduction)
         meta, hq, hkv, d, dtype = TPRPrefixMeta.shared_prefix(100, [1300, 1300, 70, 2400]), 4, 1, 256, torch.bfloat16
         assert int(meta.plan(hq, hkv, d, dtype, cuda_device).host[25]) > 0
-    else:  # bf16 with head_dim 96 runs the SIMT kernels
+    else:  # bf16 with head_dim 96 runs the general kernels
         meta, hq, hkv, d, dtype = TPRPrefixMeta.shared_prefix(96, [40, 17, 33]), 4, 2, 96, torch.bfloat16
     scale = 1.0 / math.sqrt(d)
     q, k, v, pk, pv, dout = make_inputs(meta, hq, hkv, d, dtype, 31, cuda_device)

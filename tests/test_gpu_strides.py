@@ -7,7 +7,7 @@ copy; out, lse and every gradient (into the fused projection through
 autograd) equal those of packed copies of the same values bit for bit, on
 each kernel path: head_dim 128 (32x32x16 MFMA), 64 and 256 (16x16x32 MFMA),
 at 128 and 256 with both dQ plans (the dS store, and recomputing), and the
-SIMT kernels (fp32, and bf16 at head_dim 96). The leaves mix full and
+general kernels (fp32, and bf16 at head_dim 96). The leaves mix full and
 partial 64-row tiles and suffixes longer than one dK/dV tile, so both copy
 forms of each kernel (whole tiles and the clamped tail) read through the
 stride.

@@ -229,7 +229,7 @@ def test_suffix_tiles_pair_with_their_mirror(d, kt):
 
 
 def test_suffix_tiles_stay_single_where_dkdv_workgroups_share_a_cu():
-    """head_dim 64 (several dK/dV workgroups per CU) and the SIMT kernels."""
+    """head_dim 64 (several dK/dV workgroups per CU) and the general kernels."""
     meta = TPRPrefixMeta.shared_prefix(64, [1000, 700])
     for d, dtype, path in ((64, torch.bfloat16, "mfma"), (128, torch.float32, "simt"),
                            (96, torch.bfloat16, "simt"), (256, torch.float32, "simt")):
@@ -379,7 +379,7 @@ def test_planner_rejects_unknown_plan_flags():
 
 @pytest.mark.parametrize("dtype, d", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 96)])
 def test_masked_plan_runs_simt_items_over_every_suffix_key(dtype, d):
-    """A masked plan (the mask the only visibility rule) runs the SIMT
+    """A masked plan (the mask the only visibility rule) runs the general
     kernels whatever the dtype and head size, records the longest key
     sequence as the least mask row length, gives every suffix tile's dK/dV
     item all of its leaf's query blocks (a mask may show later keys), and

@@ -54,14 +54,24 @@ def check(plan):
     return len(items)
 
 
+def tree_plan(seed, d):
+    """A random tree with every leaf four times as long, at a few head layouts."""
+    m = random_meta(500 + seed, deep=seed % 3 == 2)
+    meta = TPRPrefixMeta(tuple(4 * x for x in m.cu_seqlens_q), m.node_offsets, m.leaf_ancestors)
+    return meta.plan(*[(32, 8), (16, 4), (16, 2), (12, 3)][seed % 4], d, torch.bfloat16, CPU)
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("seed", range(12))
 def test_parts_stream_the_whole_items_blocks(seed, d):
-    m = random_meta(500 + seed, deep=seed % 3 == 2)
-    meta = TPRPrefixMeta(tuple(25 * x for x in m.cu_seqlens_q), m.node_offsets, m.leaf_ancestors)
-    plan = meta.plan(*[(8, 2), (4, 4), (6, 2), (6, 3)][seed % 4], d, torch.bfloat16, CPU)
-    if plan.host[N_KPART]:
-        check(plan)
+    plan = tree_plan(seed, d)
+    if not plan.host[N_KPART]:
+        pytest.skip("no parts in this plan")
+    check(plan)
+
+
+def test_the_random_trees_have_parts():
+    assert sum(int(tree_plan(seed, d).host[N_KPART]) > 0 for seed in range(12) for d in (64, 128, 256)) >= 34
 
 
 @pytest.mark.parametrize("d, hq, hkv", [(128, 32, 8), (64, 32, 8), (256, 8, 2), (128, 6, 3)])
