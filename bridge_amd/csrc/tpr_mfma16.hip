@@ -1039,13 +1039,17 @@ __global__ __launch_bounds__(64 * m16_dkdv_waves(kD)) void m16_dkdv(KernelArgs a
   constexpr int kKeys = m16_keys(kD);
   // head_dim 256: two waves share 16 keys, two waves a SIMD. Each takes 32 of a
   // block's 64 queries in the S / dP products and 128 of the 256 columns of dK
-  // and dV, and they hand each other P and dS through LDS. One wave for 16 keys
-  // (one a SIMD) waited on its own LDS reads, 128 KB a stage at 35 to 51 bytes a
-  // cycle beside 2048 cycles of MFMA; now the unit's 512 KB of LDS reads a stage
-  // bound it. A layer pass at prefix 4096 + 4 x 4096, GQA 8/2: 3385 -> 3177 us,
-  // its dK/dV 2217 -> 1914.
+  // and dV, and they hand each other P and dS through LDS, behind a barrier that
+  // every wave passes, keys or not. One wave for 16 keys (one a SIMD) waited on
+  // its own LDS reads, 128 KB a stage at 35 to 51 bytes a cycle beside 2048
+  // cycles of MFMA. Counters, one wave -> two: MFMA busy 32 -> 37%, LDS active
+  // 35 -> 45% of a unit's cycles, 31% of wave cycles at waits and barriers and
+  // 35% waiting to issue: no unit is full, the two barriers a stage and the
+  // waves in step are what is left. At prefix 4096 + 4 x 4096, GQA 8/2: dK/dV
+  // 2217 -> 1914 us; the layer's pass 3385 -> 3177, 3460 -> 3268 and 3541 ->
+  // 3304 us on three boxes.
   // (Four waves, two sharing 32 keys: half the LDS reads, but one wave a SIMD
-  // again, 3584 us.)
+  // again, dK/dV 2354 us.)
   constexpr bool kShare = kD == 256;
   constexpr int kW = m16_dkdv_waves(kD);
   static_assert(!kShare || kWaveKeys == 16, "one 16-key block per pair of waves");
@@ -1263,88 +1267,88 @@ __global__ __launch_bounds__(64 * m16_dkdv_waves(kD)) void m16_dkdv(KernelArgs a
             __builtin_amdgcn_sched_barrier(0);
           });
         } else {
-        // The stage is one fixed sequence of slots, each fenced: per query-block
-        // pair t, the S / dP slots (e = 0, 1; k-steps s) and then the dV / dK
-        // slots (head-dim blocks db). Every slot takes two operands from LDS
-        // (Q and dO rows, or dO and Q read transposed), and those reads are
-        // issued kRead slots ahead of the slot that uses them, so the MFMAs do
-        // not wait on LDS latency; the softmax of block (t, e) runs after its
-        // last S / dP slot, and its statistics are read at the block's first.
-        constexpr int kSD = 2 * T::NS;       // S / dP slots per t
-        constexpr int kPT = kSD + T::ND;     // slots per t
-        constexpr int kSlots = 2 * kPT;
-        constexpr int kRead = 4, kRing = kRead + 1;
-        bf16x8 ra[kRing], rb[kRing];         // slot i's operands sit at i % kRing
-        auto read_slot = [&](auto ic) __attribute__((always_inline)) {
-          constexpr int i = decltype(ic)::value;
-          constexpr int t = i / kPT, j = i % kPT;
-          if constexpr (j < kSD) {
-            constexpr int b = 2 * t + j / T::NS, s = j % T::NS;
-            ra[i % kRing] = row_operand<kD>(qt, b, s, lane);
-            rb[i % kRing] = row_operand<kD>(gt, b, s, lane);
-          } else {
-            constexpr int db = j - kSD;
-            ra[i % kRing] = col_operand<kD>(gt, 32 * t, 16 * db, lane);
-            rb[i % kRing] = col_operand<kD>(qt, 32 * t, 16 * db, lane);
-          }
-        };
-        static_for<kRead>([&](auto ic) { read_slot(ic); });
-        f32x4 sa[KB], pa[KB];
-        f32x4 ls, dl;                                  // -lse*log2e, -delta of the block's queries
-        float pf[KB][2][4], df[KB][2][4];              // [key block][query block 2t + e][register]
-        static_for<kSlots>([&](auto ic) {
-          constexpr int i = decltype(ic)::value;
-          constexpr int t = i / kPT, j = i % kPT;
-          if constexpr (i + kRead < kSlots) read_slot(std::integral_constant<int, i + kRead>{});
-          if constexpr (j < kSD) {
-            constexpr int e = j / T::NS, s = j % T::NS;
-            if constexpr (s == 0) {
-#pragma unroll
-              for (int kb = 0; kb < KB; kb++) {
-                sa[kb] = f32x4{};
-                pa[kb] = f32x4{};
-              }
-              // register r: query 32 t + 8 g + 4 e + r of the block
-              ls = *reinterpret_cast<const f32x4*>(nlse + 32 * t + 8 * g + 4 * e);
-              dl = *reinterpret_cast<const f32x4*>(ndel + 32 * t + 8 * g + 4 * e);
+          // The stage is one fixed sequence of slots, each fenced: per query-block
+          // pair t, the S / dP slots (e = 0, 1; k-steps s) and then the dV / dK
+          // slots (head-dim blocks db). Every slot takes two operands from LDS
+          // (Q and dO rows, or dO and Q read transposed), and those reads are
+          // issued kRead slots ahead of the slot that uses them, so the MFMAs do
+          // not wait on LDS latency; the softmax of block (t, e) runs after its
+          // last S / dP slot, and its statistics are read at the block's first.
+          constexpr int kSD = 2 * T::NS;       // S / dP slots per t
+          constexpr int kPT = kSD + T::ND;     // slots per t
+          constexpr int kSlots = 2 * kPT;
+          constexpr int kRead = 4, kRing = kRead + 1;
+          bf16x8 ra[kRing], rb[kRing];         // slot i's operands sit at i % kRing
+          auto read_slot = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            constexpr int t = i / kPT, j = i % kPT;
+            if constexpr (j < kSD) {
+              constexpr int b = 2 * t + j / T::NS, s = j % T::NS;
+              ra[i % kRing] = row_operand<kD>(qt, b, s, lane);
+              rb[i % kRing] = row_operand<kD>(gt, b, s, lane);
+            } else {
+              constexpr int db = j - kSD;
+              ra[i % kRing] = col_operand<kD>(gt, 32 * t, 16 * db, lane);
+              rb[i % kRing] = col_operand<kD>(qt, 32 * t, 16 * db, lane);
             }
-#pragma unroll
-            for (int kb = 0; kb < KB; kb++) {
-              sa[kb] = mfma16(ra[i % kRing], kv[kb][s], sa[kb]);
-              pa[kb] = mfma16(rb[i % kRing], vv[kb][s], pa[kb]);
-            }
-            if constexpr (s == T::NS - 1) {
-              const int q0 = 32 * t + 8 * g + 4 * e;
-#pragma unroll
-              for (int kb = 0; kb < KB; kb++) {
-                const int kp = kw0 + 16 * kb + i16;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                  float x = fmaf(sa[kb][r], c2, ls[r]);
-                  if (diag) x = kp <= tok0 + q0 + r ? x : -INFINITY;
-                  pf[kb][e][r] = fast_exp2(x);
-                  df[kb][e][r] = pf[kb][e][r] * (pa[kb][r] + dl[r]);
-                }
-              }
-              if constexpr (e == 1) {
+          };
+          static_for<kRead>([&](auto ic) { read_slot(ic); });
+          f32x4 sa[KB], pa[KB];
+          f32x4 ls, dl;                                  // -lse*log2e, -delta of the block's queries
+          float pf[KB][2][4], df[KB][2][4];              // [key block][query block 2t + e][register]
+          static_for<kSlots>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            constexpr int t = i / kPT, j = i % kPT;
+            if constexpr (i + kRead < kSlots) read_slot(std::integral_constant<int, i + kRead>{});
+            if constexpr (j < kSD) {
+              constexpr int e = j / T::NS, s = j % T::NS;
+              if constexpr (s == 0) {
 #pragma unroll
                 for (int kb = 0; kb < KB; kb++) {
-                  pT[kb] = pack8(pf[kb][0], pf[kb][1]);
-                  dT[kb] = pack8(df[kb][0], df[kb][1]);
+                  sa[kb] = f32x4{};
+                  pa[kb] = f32x4{};
+                }
+                // register r: query 32 t + 8 g + 4 e + r of the block
+                ls = *reinterpret_cast<const f32x4*>(nlse + 32 * t + 8 * g + 4 * e);
+                dl = *reinterpret_cast<const f32x4*>(ndel + 32 * t + 8 * g + 4 * e);
+              }
+#pragma unroll
+              for (int kb = 0; kb < KB; kb++) {
+                sa[kb] = mfma16(ra[i % kRing], kv[kb][s], sa[kb]);
+                pa[kb] = mfma16(rb[i % kRing], vv[kb][s], pa[kb]);
+              }
+              if constexpr (s == T::NS - 1) {
+                const int q0 = 32 * t + 8 * g + 4 * e;
+#pragma unroll
+                for (int kb = 0; kb < KB; kb++) {
+                  const int kp = kw0 + 16 * kb + i16;
+#pragma unroll
+                  for (int r = 0; r < 4; r++) {
+                    float x = fmaf(sa[kb][r], c2, ls[r]);
+                    if (diag) x = kp <= tok0 + q0 + r ? x : -INFINITY;
+                    pf[kb][e][r] = fast_exp2(x);
+                    df[kb][e][r] = pf[kb][e][r] * (pa[kb][r] + dl[r]);
+                  }
+                }
+                if constexpr (e == 1) {
+#pragma unroll
+                  for (int kb = 0; kb < KB; kb++) {
+                    pT[kb] = pack8(pf[kb][0], pf[kb][1]);
+                    dT[kb] = pack8(df[kb][0], df[kb][1]);
+                  }
                 }
               }
-            }
-          } else {
-            constexpr int db = j - kSD;
+            } else {
+              constexpr int db = j - kSD;
 #pragma unroll
-            for (int kb = 0; kb < KB; kb++) {
-              dv[kb][db] = mfma16(pT[kb], ra[i % kRing], dv[kb][db]);
-              dk[kb][db] = mfma16(dT[kb], rb[i % kRing], dk[kb][db]);
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        });
+              for (int kb = 0; kb < KB; kb++) {
+                dv[kb][db] = mfma16(pT[kb], ra[i % kRing], dv[kb][db]);
+                dk[kb][db] = mfma16(dT[kb], rb[i % kRing], dk[kb][db]);
               }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        }
       } else if constexpr (kShare) {
         asm volatile("s_barrier" ::: "memory");  // the hand-over's
       }

@@ -291,7 +291,10 @@ class TPRPrefixAttention(torch.autograd.Function):
     prefix_state.py:546-573, in fp32 and inside the kernel) and gives
     prefix_k / prefix_v no autograd gradient; they must then not require one.
 
-    Memory: the backward's workspace holds, besides a few MB of statistics,
+    Memory: the forward of few query rows takes up to 192 MiB for its key
+    parts, given back before it returns. The backward's workspace holds,
+    besides a few MB of statistics and, where few rows or key tiles are cut
+    over more workgroups, up to 192 MiB of dQ and 134 MB of dK/dV partials,
     the dS store when the plan has one -- 2 bytes per visible (query, key)
     pair and query head, 6.5 GB at the Qwen3-4B layer shape (prefix 4096 +
     4 x 4096, GQA 32/8) -- which makes dQ one matrix product instead of three.
