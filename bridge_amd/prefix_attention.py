@@ -205,18 +205,18 @@ def _check_accumulators(accumulators, prefix_k) -> Tuple[torch.Tensor, torch.Ten
     return accumulators[0], accumulators[1]
 
 
-def _allocate(plan, device, must):
+def _allocate(plan, device):
     """(workspace, its bytes) for a plan's backward: the full size, or the least
-    where that does not fit. Where neither does: None, or with ``must`` the
-    allocator's error. The error is never held: a caught exception kept in a
-    local would keep the callers' frames, and every tensor in them, until the
-    cyclic collector runs."""
+    where that does not fit. Where neither does: None for a plan with a dS
+    store, else the allocator's error. The error is never held: a caught
+    exception kept in a local would keep the callers' frames, and every tensor
+    in them, until the cyclic collector runs."""
     least = plan.workspace_bytes if plan.bwd_min_bytes is None else plan.bwd_min_bytes
     for size in sorted({plan.workspace_bytes, least}, reverse=True):
         try:
             return torch.empty(size, dtype=torch.uint8, device=device) if size else None, size
         except torch.OutOfMemoryError:
-            if must and size == least:
+            if size == least and not plan.dq_from_ds:
                 raise
     return None
 
@@ -232,10 +232,10 @@ def _workspace(meta, q, k, budget, ws, masked=False):
     if ws is not None:
         behind = ws.untyped_storage().nbytes() - ws.storage_offset() * ws.element_size()
         return plan, ws, min(ws.numel() * ws.element_size(), behind)
-    got = _allocate(plan, q.device, must=not plan.dq_from_ds)
+    got = _allocate(plan, q.device)
     if got is None:
         plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, ds_store_budget=0)
-        got = _allocate(plan, q.device, must=True)
+        got = _allocate(plan, q.device)
     return plan, *got
 
 
