@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+from unittest import mock
 
 import pytest
 import torch
@@ -73,6 +74,35 @@ def test_key_parts_match_oracle_and_whole_items(name, d, recompute, strided, cud
     # every row on its own: a part added twice or left out hides in a norm over all rows
     err = (out.double().cpu() - ro).norm(dim=2) / ro.norm(dim=2)
     assert err.max().item() <= 3 * BF16_REL
+
+
+def test_forward_without_memory_for_its_parts_runs_whole_items(cuda_device):
+    """The workspace cannot be allocated (host side, forced): the result is that
+    of the call without one, bit for bit, with and without a backward to follow."""
+    from bridge_amd import TPRPrefixMeta, _lib, prefix_attention_forward, tpr_prefix_attention
+    meta, d = TPRPrefixMeta.shared_prefix(1500, [100]), 128
+    plan = meta.plan(32, 8, d, torch.bfloat16, cuda_device)
+    q, k, v, pk, pv, _ = make_inputs(meta, 32, 8, d, torch.bfloat16, seed=2, device=cuda_device)
+    whole, whole_lse = torch.empty_like(q), torch.empty(32, 100, dtype=torch.float32, device=cuda_device)
+    params = _lib.TprFwdParams(_lib.ABI_VERSION, 0, 1.0 / math.sqrt(d), 0.0, plan.host.data_ptr(), plan.device.data_ptr(),
+                               *(t.data_ptr() for t in (q, k, v, pk, pv, whole, whole_lse)), 0, 0, 0, None, 0)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(cuda_device).cuda_stream)
+    _lib.check(_lib.load().tpr_attn_fwd(ctypes.byref(params), stream), "tpr_attn_fwd")
+    real, asked = torch.empty, []
+
+    def empty(size, *args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8:
+            asked.append(size)
+            raise torch.OutOfMemoryError("no memory")
+        return real(size, *args, **kwargs)
+
+    with mock.patch.object(torch, "empty", empty):
+        out, lse = prefix_attention_forward(q, k, v, pk, pv, meta)
+        leaf = q.clone().requires_grad_(True)
+        out2, _ = tpr_prefix_attention(leaf, k, v, pk, pv, meta)
+    torch.cuda.synchronize()
+    assert asked == [plan.fwd_workspace_bytes, plan.workspace_bytes, plan.fwd_workspace_bytes]
+    assert torch.equal(out, whole) and torch.equal(out2, whole) and torch.equal(lse, whole_lse)
 
 
 def test_key_parts_are_deterministic_and_replay(cuda_device):
