@@ -61,6 +61,8 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     """``t`` itself when the kernels can read it through a row stride (heads
     and head_dim packed, rows 16-byte aligned: a slice of a fused
     [tokens, (Hq + 2 Hkv) * D] projection is one), else a packed copy."""
+    if t.is_contiguous():
+        return t
     _, h, d = t.shape
     es = t.element_size()
     rs = t.stride(0)
@@ -72,6 +74,8 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
 
 def _row_stride(t: torch.Tensor) -> int:
     """Row stride (elements) for the ABI: 0 when packed."""
+    if t.is_contiguous():
+        return 0
     _, h, d = t.shape
     return 0 if t.shape[0] <= 1 or t.stride(0) == h * d else t.stride(0)
 
@@ -96,28 +100,29 @@ def validate(q, k, v, prefix_k, prefix_v, meta: TPRPrefixMeta, softmax_scale):
     if not isinstance(meta, TPRPrefixMeta):
         raise TypeError(f"meta must be a TPRPrefixMeta, got {type(meta).__name__}")
     tq, hq, d = q.shape
-    if k.shape != v.shape:
+    k_shape, p_shape = k.shape, prefix_k.shape
+    if k_shape != v.shape:
         raise ValueError(f"key and value must have identical shapes, got key={tuple(k.shape)}, value={tuple(v.shape)}")
-    if prefix_k.shape != prefix_v.shape:
+    if p_shape != prefix_v.shape:
         raise ValueError("prefix key and value must have identical shapes, "
                          f"got key={tuple(prefix_k.shape)}, value={tuple(prefix_v.shape)}")
-    hkv = k.shape[1]
-    if k.shape[0] != tq:
+    tk, hkv, dk = k_shape
+    tp, hp, dp = p_shape
+    if tk != tq:
         raise ValueError(f"suffix key length must equal query length, got Q={tq}, KV={k.shape[0]}")
-    if k.shape[2] != d or prefix_k.shape[2] != d:
+    if dk != d or dp != d:
         raise ValueError(f"Q and KV head dimensions must match, got Q={d}, KV={k.shape[2]}, prefix={prefix_k.shape[2]}")
-    if prefix_k.shape[1] != hkv:
+    if hp != hkv:
         raise ValueError(f"prefix KV head count must match suffix KV heads, got {prefix_k.shape[1]} vs {hkv}")
     if hq <= 0 or hkv <= 0 or d <= 0:
         raise ValueError(f"head counts and head_dim must be positive, got Q={tuple(q.shape)}, KV={tuple(k.shape)}")
     if hq % hkv != 0:
         raise ValueError(f"query head count must be divisible by KV head count, got Q={hq}, KV={hkv}")
-    dtypes = {q.dtype, k.dtype, v.dtype, prefix_k.dtype, prefix_v.dtype}
-    if len(dtypes) != 1:
+    if not q.dtype == k.dtype == v.dtype == prefix_k.dtype == prefix_v.dtype:
         raise ValueError(f"Q, K, and V dtypes must match, got Q={q.dtype}, K={k.dtype}, V={v.dtype}, "
                          f"prefix K={prefix_k.dtype}, prefix V={prefix_v.dtype}")
-    devices = {q.device, k.device, v.device, prefix_k.device, prefix_v.device}
-    if len(devices) != 1:
+    if not q.device == k.device == v.device == prefix_k.device == prefix_v.device:
+        devices = {q.device, k.device, v.device, prefix_k.device, prefix_v.device}
         raise ValueError(f"Q, K, and V devices must match, got {sorted(str(x) for x in devices)}")
     if not q.is_floating_point():
         raise ValueError(f"Q, K, and V must use a floating-point dtype, got {q.dtype}")
@@ -125,7 +130,7 @@ def validate(q, k, v, prefix_k, prefix_v, meta: TPRPrefixMeta, softmax_scale):
         raise ValueError(f"prefix attention supports torch.bfloat16 and torch.float32, got {q.dtype}")
     if tq != meta.total_q:
         raise ValueError(f"query rows ({tq}) must equal meta.total_q ({meta.total_q})")
-    if prefix_k.shape[0] != meta.total_prefix:
+    if tp != meta.total_prefix:
         raise ValueError(f"prefix rows ({prefix_k.shape[0]}) must equal meta.total_prefix ({meta.total_prefix})")
     if q.device.type != "cuda":
         raise RuntimeError(f"tpr_prefix_attention requires a ROCm GPU (cuda) tensor, got device {q.device}")
