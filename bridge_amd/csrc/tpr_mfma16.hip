@@ -1047,7 +1047,7 @@ __global__ __launch_bounds__(64 * m16_dkdv_waves(kD)) void m16_dkdv(KernelArgs a
   // 35% waiting to issue: no unit is full, the two barriers a stage and the
   // waves in step are what is left. At prefix 4096 + 4 x 4096, GQA 8/2: dK/dV
   // 2217 -> 1914 us; the layer's pass 3385 -> 3177, 3460 -> 3268 and 3541 ->
-  // 3304 us on three boxes.
+  // 3304 us on three machines.
   // (Four waves, two sharing 32 keys: half the LDS reads, but one wave a SIMD
   // again, dK/dV 2354 us.)
   constexpr bool kShare = kD == 256;

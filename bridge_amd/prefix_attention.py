@@ -175,8 +175,8 @@ def _forward_bytes(plan, backward):
     """Bytes to ask for as the forward's workspace. Where a backward follows,
     its size, up to 256 MiB: the allocator then keeps one block for both, which
     on the first pass of a new schedule is one call of the driver (100 us)
-    instead of two (prefix 1500 + 100, GQA 32/8, d128: 625 -> 495 us, on another
-    box 519 -> 430)."""
+    instead of two (prefix 1500 + 100, GQA 32/8, d128: 625 -> 495 us; on
+    another machine 519 -> 430)."""
     if plan.fwd_workspace_bytes and backward and plan.workspace_bytes <= _ONE_SIZE_BYTES:
         return max(plan.fwd_workspace_bytes, plan.workspace_bytes)
     return plan.fwd_workspace_bytes
