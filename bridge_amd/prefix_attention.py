@@ -168,21 +168,7 @@ def _mask_args(mask: Optional[torch.Tensor]) -> Tuple[Optional[int], int]:
     return _ptr(mask), int(mask.shape[1])
 
 
-_ONE_SIZE_BYTES = 256 << 20
-
-
-def _forward_bytes(plan, backward):
-    """Bytes to ask for as the forward's workspace. Where a backward follows,
-    its size, up to 256 MiB: the allocator then keeps one block for both, which
-    on the first pass of a new schedule is one call of the driver (100 us)
-    instead of two (prefix 1500 + 100, GQA 32/8, d128: 625 -> 495 us; on
-    another machine 519 -> 430)."""
-    if plan.fwd_workspace_bytes and backward and plan.workspace_bytes <= _ONE_SIZE_BYTES:
-        return max(plan.fwd_workspace_bytes, plan.workspace_bytes)
-    return plan.fwd_workspace_bytes
-
-
-def _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask=None, backward=False):
+def _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask=None):
     plan = meta.plan(q.shape[1], k.shape[1], q.shape[2], q.dtype, q.device, masked=mask is not None)
     out = _empty(q)
     lse = torch.empty((q.shape[1], q.shape[0]), dtype=torch.float32, device=q.device)
@@ -194,13 +180,12 @@ def _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask=None, backward=False
         plan.host.data_ptr(), plan.device.data_ptr(),
         _ptr(q), _ptr(k), _ptr(v), _ptr(prefix_k), _ptr(prefix_v), _ptr(out), _ptr(lse),
         _row_stride(q), _row_stride(k), _row_stride(v), *_mask_args(mask))
-    ws = None  # where none can be allocated the forward runs without key parts
-    for size in sorted({_forward_bytes(plan, backward), plan.fwd_workspace_bytes} - {0}, reverse=True):
+    ws = None
+    if plan.fwd_workspace_bytes:
         try:
-            ws = torch.empty(size, dtype=torch.uint8, device=q.device)
-            break
+            ws = torch.empty(plan.fwd_workspace_bytes, dtype=torch.uint8, device=q.device)
         except torch.OutOfMemoryError:
-            pass
+            pass  # the forward runs without key parts
     _lib.check(lib.tpr_attn_fwd_ws(ctypes.byref(params), _ptr(ws), plan.fwd_workspace_bytes,
                                    ctypes.c_void_p(_stream_handle(q.device))), "tpr_attn_fwd")
     return out, lse
@@ -312,8 +297,7 @@ class TPRPrefixAttention(torch.autograd.Function):
     prefix_k / prefix_v no autograd gradient; they must then not require one.
 
     Memory: the forward of few query rows takes up to 192 MiB for its key
-    parts (256 MiB where it asks for the backward's size), given back before it
-    returns. The backward's workspace holds,
+    parts, given back before it returns. The backward's workspace holds,
     besides a few MB of statistics and, where few rows or key tiles are cut
     over more workgroups, up to 192 MiB of dQ and 134 MB of dK/dV partials,
     the dS store when the plan has one -- 2 bytes per visible (query, key)
@@ -339,7 +323,7 @@ class TPRPrefixAttention(torch.autograd.Function):
                 raise ValueError("prefix_k/prefix_v must not require grad when prefix_grad_accumulators is given")
             _check_accumulators(prefix_grad_accumulators, prefix_k)
         q, k, v, prefix_k, prefix_v = _inputs(q, k, v, prefix_k, prefix_v)
-        out, lse = _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask, any(ctx.needs_input_grad))
+        out, lse = _forward(q, k, v, prefix_k, prefix_v, meta, scale, mask)
         ctx.save_for_backward(q, k, v, prefix_k, prefix_v, out, lse)
         ctx.mask = mask
         ctx.meta = meta

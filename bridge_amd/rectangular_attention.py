@@ -115,7 +115,7 @@ class _RectangularAttention(torch.autograd.Function):
         scale = validate(*rows, meta, scale)
         mask = check_mask(attention_mask, q, meta)
         rows = _inputs(*rows)
-        out, lse = _forward(*rows, meta, scale, mask, any(ctx.needs_input_grad))
+        out, lse = _forward(*rows, meta, scale, mask)
         ctx.save_for_backward(*rows, out, lse)
         ctx.mask, ctx.meta, ctx.scale = mask, meta, scale
         return out

@@ -101,7 +101,7 @@ def test_forward_without_memory_for_its_parts_runs_whole_items(cuda_device):
         leaf = q.clone().requires_grad_(True)
         out2, _ = tpr_prefix_attention(leaf, k, v, pk, pv, meta)
     torch.cuda.synchronize()
-    assert asked == [plan.fwd_workspace_bytes, plan.workspace_bytes, plan.fwd_workspace_bytes]
+    assert asked == [plan.fwd_workspace_bytes] * 2
     assert torch.equal(out, whole) and torch.equal(out2, whole) and torch.equal(lse, whole_lse)
 
 

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from bridge_amd import TPRPrefixMeta, _lib
-from bridge_amd.prefix_attention import _forward_bytes, _workspace
+from bridge_amd.prefix_attention import _workspace
 
 CPU = torch.device("cpu")
 
@@ -46,20 +46,6 @@ def test_less_than_the_least_is_refused_before_a_launch(short):
         b.workspace = 4096 + 16  # enough, but misaligned: the next check
     status = _lib.load().tpr_attn_bwd(ctypes.byref(b), None)
     assert status == (_lib.TPR_ERR_BUFFER_TOO_SMALL if short else _lib.TPR_ERR_INVALID_ARGUMENT)
-
-
-def test_the_forward_asks_for_the_backwards_size():
-    """One block for both where a backward follows, never less than the forward
-    needs, and not for a large dS store."""
-    def plan(prefix, lens):
-        return TPRPrefixMeta.shared_prefix(prefix, lens).plan(32, 8, 128, torch.bfloat16, CPU)
-
-    small, large, none = plan(1500, [100]), plan(8192, [512]), plan(4096, [4096] * 4)
-    assert 0 < small.fwd_workspace_bytes < small.workspace_bytes <= 256 << 20 < large.workspace_bytes
-    assert _forward_bytes(small, True) == small.workspace_bytes
-    assert _forward_bytes(small, False) == small.fwd_workspace_bytes
-    assert _forward_bytes(large, True) == large.fwd_workspace_bytes > 0
-    assert _forward_bytes(none, True) == _forward_bytes(none, False) == 0
 
 
 def _failing_empty(fails):
